@@ -17,6 +17,7 @@
 #include "../../include/nfftm.h"
 #include "fft1.hpp"
 #include "launch.hpp"
+#include "mixfft.hpp"
 
 using namespace nfftm;
 typedef int64_t i64;
@@ -475,6 +476,9 @@ struct nfftm_plan_s {
   std::unique_ptr<FFTStage> fft;
   // pruned FFT passes (power-of-two grids): twiddle tables per dimension
   bool pfft = false;
+  // the same passes with per-plan radices (other grids): line radices
+  bool mix = false;
+  MixLine mixln[3];
   DevBuf<char> d_tw;
   size_t tw_off[3] = {0, 0, 0};
   // 1-D grids of n1 Lm^2 points: the three-pass FFT of k_fft1.hip, its
@@ -633,6 +637,63 @@ struct nfftm_plan_s {
     }
     a.oscale = 1.0;
     a.ist = io_stride;
+    return a;
+  }
+
+  // Pass over the lines of dimension d (k_mixfft.hip).
+  MixArgs mixargs(int d) const {
+    MixArgs a;
+    std::memset(&a, 0, sizeof a);
+    i64 n[3] = {1, 1, 1}, l[3] = {1, 1, 1}, na[3] = {0, 0, 0}, gs[4] = {1, 1, 1, 1}, off = 0;
+    for (int e = 0; e < 3; ++e) {
+      if (e < D) {
+        n[e] = N[e];
+        l[e] = Nt[e];
+        na[e] = N[e] / 2;
+        a.fac[e] = d_deconv.p + off;
+        off += N[e];
+      }
+      gs[e + 1] = gs[e] * l[e];
+    }
+    a.ln = mixln[d];
+    a.tw = d_tw.p + tw_off[d];
+    a.N = (int)n[d];
+    a.Na = (int)na[d];
+    a.st = gs[d];
+    if (d == 0) {
+      a.nlines = (int)(n[1] * n[2]);
+      a.lpb = mix_shape(dbl(), false, a.ln, a.nlines, 1);
+      a.total = (a.nlines + a.lpb - 1) / a.lpb;
+    } else {
+      const int o = 3 - d;
+      a.oall = d == 2;
+      a.oN = (int)n[o];
+      a.oL = (int)l[o];
+      a.oNa = (int)na[o];
+      a.ost = gs[o];
+      a.nx = (int)l[0];
+      const i64 outer = a.oall ? l[o] : n[o];
+      a.lpb = mix_shape(dbl(), true, a.ln, a.nx, outer);
+      a.nchunk = (a.nx + a.lpb - 1) / a.lpb;
+      a.total = (int)(a.nchunk * outer);
+    }
+    while ((1 << a.lsh) < a.lpb) ++a.lsh;
+    a.dchunk = make_fastdiv((uint32_t)std::max(1, a.nchunk));
+    a.dN1 = make_fastdiv((uint32_t)n[1]);
+    a.N1 = (int)n[1];
+    a.L1 = (int)l[1];
+    a.Na1 = (int)na[1];
+    a.st1 = gs[1];
+    a.N2 = (int)n[2];
+    a.L2 = (int)l[2];
+    a.Na2 = (int)na[2];
+    a.st2 = gs[2];
+    a.oscale = 1.0;
+    a.ist = io_stride;
+    a.nsl = 1;
+    a.Bsl = 1;
+    a.P = P;
+    a.Q = Q;
     return a;
   }
 
@@ -1136,6 +1197,16 @@ int forward_to_grid(nfftm_plan_s& p, const void* f, Mark&& mark) {
     HIPCHK(launch_pruned_fft_fwd(p.dbl(), a, p.stream, f, p.d_grid.p, 1));
     return NFFTM_OK;
   }
+  if (p.mix) {
+    {
+      ProfScope ps(p, 0);
+      HIPCHK(launch_mix_x(p.dbl(), true, p.mixargs(0), p.stream, f, p.d_grid.p));
+    }
+    if (int rc = mark()) return rc;
+    ProfScope ps(p, 1);
+    for (int d = 1; d < p.D; ++d) HIPCHK(launch_mix_col(p.dbl(), true, p.mixargs(d), p.stream, p.d_grid.p));
+    return NFFTM_OK;
+  }
   if (p.f1) {
     const F1Args a = p.f1args();
     {
@@ -1171,6 +1242,16 @@ int grid_to_image(nfftm_plan_s& p, void* f, Mark&& mark, bool fused = false) {
     if (int rc = mark()) return rc;
     ProfScope ps(p, 6);
     HIPCHK(launch_pruned_fft_adj(p.dbl(), a, p.stream, p.d_grid.p, f, 1));
+    return NFFTM_OK;
+  }
+  if (p.mix) {
+    {
+      ProfScope ps(p, 5);
+      for (int d = p.D - 1; d >= 1; --d) HIPCHK(launch_mix_col(p.dbl(), false, p.mixargs(d), p.stream, p.d_grid.p));
+    }
+    if (int rc = mark()) return rc;
+    ProfScope ps(p, 6);
+    HIPCHK(launch_mix_x(p.dbl(), false, p.mixargs(0), p.stream, p.d_grid.p, f));
     return NFFTM_OK;
   }
   if (p.f1) {
@@ -1247,7 +1328,10 @@ int create_impl(nfftm_plan_s& p, const double* k) {
   p.fft.reset(new FFTStage());
   if (int rc = p.fft->build(p.D, p.Nt, p.dbl())) return rc;
   p.pfft = !(p.flags & NFFTM_FLAG_ROCFFT) && pruned_fft_supported(p.D, p.N, p.Nt, p.dbl());
-  if (p.pfft) {
+  p.mix = !(p.flags & NFFTM_FLAG_ROCFFT) && !p.pfft && p.D <= 3 && p.Q < (1LL << 31);
+  for (int d = 0; d < p.D && p.mix; ++d)
+    p.mix = p.N[d] <= p.Nt[d] && mix_factor(p.Nt[d], p.dbl(), p.D == 1, &p.mixln[d]);
+  if (p.pfft || p.mix) {
     // twiddle tables exp(-2 pi i k / Nt_d) as (cos, sin) of 2 pi k / Nt_d,
     // FP64 on the host, stored in the data precision
     const size_t es = p.dbl() ? 16 : 8;
@@ -1275,7 +1359,7 @@ int create_impl(nfftm_plan_s& p, const double* k) {
     HIPCHK(p.d_tw.alloc(bytes));
     HIPCHK(hipMemcpy(p.d_tw.p, h.data(), bytes, hipMemcpyHostToDevice));
   }
-  p.f1 = !p.pfft && p.D == 1 && !(p.flags & NFFTM_FLAG_ROCFFT) &&
+  p.f1 = !p.pfft && !p.mix && p.D == 1 && !(p.flags & NFFTM_FLAG_ROCFFT) &&
          fft1_factor(p.Nt[0], p.N[0], p.dbl(), &p.f1n1, &p.f1Lm);
   if (p.f1) {
     // (cos, sin)(2 pi j / n1) and (2 pi j / Lm) in the data precision,
