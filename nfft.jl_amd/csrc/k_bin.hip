@@ -76,27 +76,28 @@ __global__ __launch_bounds__(BT) void k_bin_keys_lds(BinArgs a, const double* __
 
 // One workgroup: off = exclusive scan of cnt (ntile + 1 entries), ioff =
 // exclusive scan of ceil(cnt / CH) (work items per tile); stats[0] = number
-// of work items, stats[1] = most items of one tile.
+// of work items, stats[1] = tiles of more than one, stats[2] = 0 (the counter
+// of k_bin_items).
 constexpr int ST = 1024;
 __global__ __launch_bounds__(ST) void k_bin_scan(BinArgs a, const int* __restrict__ cnt, int* __restrict__ off,
                                                  int* __restrict__ ioff, int* __restrict__ stats) {
   __shared__ long long s_n[ST], s_i[ST];
-  __shared__ int s_max[ST];
+  __shared__ int s_mul[ST];
   const int n = a.ntile;
   const int per = (n + ST - 1) / ST;
   const int b = threadIdx.x * per, e = min(n, b + per);
   long long sn = 0, si = 0;
-  int mx = 0;
+  int mx = 0;  // tiles of several items
   for (int t = b; t < e; ++t) {
     const int c = cnt[t];
     const int it = (c + a.CH - 1) / a.CH;
     sn += c;
     si += it;
-    mx = max(mx, it);
+    mx += it > 1;
   }
   s_n[threadIdx.x] = sn;
   s_i[threadIdx.x] = si;
-  s_max[threadIdx.x] = mx;
+  s_mul[threadIdx.x] = mx;
   __syncthreads();
   if (threadIdx.x == 0) {  // ST partial sums: serial exclusive scan
     long long an = 0, ai = 0;
@@ -107,12 +108,13 @@ __global__ __launch_bounds__(ST) void k_bin_scan(BinArgs a, const int* __restric
       s_i[w] = ai;
       an += tn;
       ai += ti;
-      am = max(am, s_max[w]);
+      am += s_mul[w];
     }
     off[n] = (int)an;
     ioff[n] = (int)ai;
     stats[0] = (int)ai;
     stats[1] = am;
+    stats[2] = 0;
   }
   __syncthreads();
   long long an = s_n[threadIdx.x], ai = s_i[threadIdx.x];
@@ -126,15 +128,18 @@ __global__ __launch_bounds__(ST) void k_bin_scan(BinArgs a, const int* __restric
 }
 
 // Work items of tile t: {t, begin, end, 0} for chunks of at most CH nodes;
-// tstart[t] = first item of tile t (tstart[ntile] = number of items).
+// tstart[t] = first item of tile t (tstart[ntile] = number of items); the
+// tiles of several items are listed in multi (in any order).
 __global__ __launch_bounds__(BT) void k_bin_items(BinArgs a, const int* __restrict__ off, const int* __restrict__ ioff,
-                                                  int4* __restrict__ items, int* __restrict__ tstart) {
+                                                  int4* __restrict__ items, int* __restrict__ tstart,
+                                                  int* __restrict__ multi, int* __restrict__ nmulti) {
   const long long t = (long long)blockIdx.x * BT + threadIdx.x;
   if (t > a.ntile) return;
   tstart[t] = ioff[t];
   if (t == a.ntile) return;
   const int b0 = off[t], e0 = off[t + 1];
   int q = ioff[t];
+  if (ioff[t + 1] - q > 1) multi[atomicAdd(nmulti, 1)] = (int)t;
   for (int s = b0; s < e0; s += a.CH) items[q++] = int4{(int)t, s, min(e0, s + a.CH), 0};
 }
 
@@ -188,9 +193,10 @@ hipError_t launch_bin_scan(const BinArgs& a, const int* cnt, int* off, int* ioff
   return hipGetLastError();
 }
 
-hipError_t launch_bin_items(const BinArgs& a, const int* off, const int* ioff, int4* items, int* tstart,
-                            hipStream_t s) {
-  hipLaunchKernelGGL(k_bin_items, dim3(blocks((long long)a.ntile + 1)), dim3(BT), 0, s, a, off, ioff, items, tstart);
+hipError_t launch_bin_items(const BinArgs& a, const int* off, const int* ioff, int4* items, int* tstart, int* multi,
+                            int* nmulti, hipStream_t s) {
+  hipLaunchKernelGGL(k_bin_items, dim3(blocks((long long)a.ntile + 1)), dim3(BT), 0, s, a, off, ioff, items, tstart,
+                     multi, nmulti);
   return hipGetLastError();
 }
 

@@ -38,8 +38,8 @@ struct FArgs {
 // Power-of-two grids within the line kernels' LDS (FP32: 16..2048 points
 // per dimension, FP64: 16..1024), D <= 3, N_d <= Nt_d.
 bool pruned_fft_supported(int D, const int64_t* N, const int64_t* Nt, bool dbl);
-// Adjoint, 3-D block-layout slots with at most one work item per tile: the
-// fold fused into the first pruned pass (dimension 3), grid positions S_z of
+// Adjoint, 3-D block-layout slots of whole tiles: the fold fused into the
+// first pruned pass (dimension 3), grid positions S_z of
 // every (x, y) line written.  hipErrorNotSupported (nothing launched) where
 // the tile geometry does not match the pass; dry = only that check.
 hipError_t launch_fold_fft3(bool dbl, int W, const KArgs& a, const FArgs& f, hipStream_t s, void* grid, bool dry);
@@ -131,8 +131,8 @@ hipError_t launch_bin_keys(const BinArgs& a, const double* k, int* key, int* idx
 hipError_t launch_bin_sort(const BinArgs& a, void* temp, size_t temp_bytes, int* key_in, int* key_out, int* idx_in,
                            int* idx_out, hipStream_t s);
 hipError_t launch_bin_scan(const BinArgs& a, const int* cnt, int* off, int* ioff, int* stats, hipStream_t s);
-hipError_t launch_bin_items(const BinArgs& a, const int* off, const int* ioff, int4* items, int* tstart,
-                            hipStream_t s);
+hipError_t launch_bin_items(const BinArgs& a, const int* off, const int* ioff, int4* items, int* tstart, int* multi,
+                            int* nmulti, hipStream_t s);
 hipError_t launch_bin_ks(const BinArgs& a, const double* k, const int* perm, double* ks, hipStream_t s);
 hipError_t launch_iota(int* p, long long n, hipStream_t s);
 
@@ -154,6 +154,9 @@ hipError_t launch_fold(int D, bool dbl, int W, const KArgs& a, hipStream_t s, vo
 hipError_t launch_sparse_build(bool dbl, int W, const KArgs& a, hipStream_t s, int* cols, void* vals);
 hipError_t launch_sparse(bool spread, bool dbl, const KArgs& a, int K, const int* cols, const void* vals,
                          hipStream_t s, const void* in, void* out);
+// 3-D: the slots of tiles with several work items (the list multi) summed
+// into the tile's first slot, which is the one the 3-D folds read.
+hipError_t launch_slot_sum(bool dbl, const KArgs& a, size_t slot_bytes, const int* multi, int nmulti, hipStream_t s);
 hipError_t launch_fold_d3(bool dbl, int W, const KArgs& a, hipStream_t s, void* grid);
 
 // Per-CU cycles of one wavefront instruction of ds_read_b64, ds_read_b128,

@@ -419,12 +419,12 @@ struct nfftm_plan_s {
   // arguments: Bsl while a directional transform runs, 1 otherwise (the
   // plan's own work vectors are contiguous)
   i64 io_stride = 1;
-  // 3-D scratch slots in halo/interior block layout: whole tiles per
-  // dimension and halos (m - 1, m cells) no wider than a tile
+  // 3-D scratch slots in halo/interior block layout: halos (m - 1, m cells)
+  // no wider than any tile, a partial last one included
   bool blocked3() const {
     if (D != 3 || !tiled) return false;
     for (int d = 0; d < 3; ++d)
-      if (Nt[d] % T[d] != 0 || T[d] < m) return false;
+      if (T[d] < m || Nt[d] - (ntiles[d] - 1) * T[d] < m) return false;
     return true;
   }
   // cells of one scratch slot (3-D: rounded to a 128-byte multiple)
@@ -464,7 +464,8 @@ struct nfftm_plan_s {
   DevBuf<int> d_bcols;
   DevBuf<char> d_bvals;
   int nitems = 0;
-  bool single_items = false;  // tiled, nitems > 0, no tile with two work items
+  DevBuf<int> d_multi;        // tiles of several work items
+  int nmulti = 0;
   int gen = 0;        // incremented whenever the node arrays are rebuilt
   double wmax = 1.0;  // bound of one (normalised) window value
 
@@ -944,7 +945,7 @@ int set_nodes(nfftm_plan_s& p, const double* k, i64 M) {
   if (M) HIPCHK(hipMemcpyAsync(kd.p, k, (size_t)D * M * sizeof(double), hipMemcpyHostToDevice, st));
   HIPCHK(p.d_ks.alloc((size_t)D * M));
   HIPCHK(p.d_perm.alloc((size_t)M));
-  int nitems = 0, most = 0;
+  int nitems = 0, nmulti = 0;
   if (!p.tiled) {
     HIPCHK(launch_iota(p.d_perm.p, M, st));
     HIPCHK(launch_bin_ks(a, kd.p, nullptr, p.d_ks.p, st));
@@ -958,7 +959,7 @@ int set_nodes(nfftm_plan_s& p, const double* k, i64 M) {
     HIPCHK(cnt.alloc((size_t)ntile + 1));
     HIPCHK(off.alloc((size_t)ntile + 1));
     HIPCHK(ioff.alloc((size_t)ntile + 1));
-    HIPCHK(stats.alloc(2));
+    HIPCHK(stats.alloc(3));
     HIPCHK(launch_bin_keys(a, kd.p, key_in.p, idx_in.p, cnt.p, st));
     DevBuf<char> tmp;
     if (M) {
@@ -972,15 +973,16 @@ int set_nodes(nfftm_plan_s& p, const double* k, i64 M) {
     HIPCHK(hipMemcpyAsync(hs, stats.p, sizeof hs, hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
     nitems = hs[0];
-    most = hs[1];
+    nmulti = hs[1];
     HIPCHK(p.d_items.alloc((size_t)nitems));
     HIPCHK(p.d_tstart.alloc((size_t)ntile + 1));
-    HIPCHK(launch_bin_items(a, off.p, ioff.p, p.d_items.p, p.d_tstart.p, st));
+    HIPCHK(p.d_multi.alloc((size_t)nmulti));
+    HIPCHK(launch_bin_items(a, off.p, ioff.p, p.d_items.p, p.d_tstart.p, p.d_multi.p, stats.p + 2, st));
     HIPCHK(launch_bin_ks(a, kd.p, p.d_perm.p, p.d_ks.p, st));
     HIPCHK(hipStreamSynchronize(st));  // before the temporaries are freed
   }
   p.nitems = nitems;
-  p.single_items = p.tiled && nitems > 0 && most <= 1;
+  p.nmulti = nmulti;
   if (p.sparse && M > 0) {
     i64 K = 1;
     for (int d = 0; d < D; ++d) K *= p.W;
@@ -1086,7 +1088,7 @@ struct ProfScope {
 bool fused_fold(const nfftm_plan_s& p) {
   if (p.flags & NFFTM_FLAG_SEPARATE_FOLD) return false;
   if (p.f1) return p.tiled && p.D == 1;
-  return p.pfft && p.blocked3() && p.single_items &&
+  return p.pfft && p.blocked3() && p.nitems > 0 && p.nmulti == 0 &&
          launch_fold_fft3(p.dbl(), p.W, p.kargs(), p.fargs(), nullptr, nullptr, true) == hipSuccess;
 }
 
@@ -1114,6 +1116,10 @@ int run_conv(nfftm_plan_s& p, bool spread, const void* in, void* out, bool stand
       e = launch_generic(spread, p.dbl(), p.W, a, p.stream, in, out);
   }
   HIPCHK(e);
+  if (spread && p.tiled && p.D == 3 && p.nmulti > 0) {
+    ProfScope ps(p, 3);
+    HIPCHK(launch_slot_sum(p.dbl(), a, p.slot_cells() * p.celem(), p.d_multi.p, p.nmulti, p.stream));
+  }
   if (spread && p.tiled && fold) {
     ProfScope ps(p, 3);
     HIPCHK(launch_fold(p.D, p.dbl(), p.W, a, p.stream, out));
