@@ -41,6 +41,11 @@ __device__ __forceinline__ double line_factor(const FArgs& a, int iy, int iz, bo
   return f;
 }
 
+// Grid of the launch's slice i (KArgs).
+__device__ __forceinline__ size_t slice_grid(const FArgs& a, int i) {
+  return (size_t)(a.nsl - 1 - i) * (size_t)a.Q;
+}
+
 // Forward, dimension 1: deconvolution of f into lines (y, z) in S_y x S_z,
 // zero padding, FFT, whole lines to the grid.
 template <typename R, int L>
@@ -56,6 +61,7 @@ __global__ __launch_bounds__((LineGeo<R, L>::NT)) void k_fft_x_fwd(FArgs a, cons
   const int nlines = a.N[1] * a.N[2];
   const int l = threadIdx.x / G::TL, j0 = threadIdx.x % G::TL;
   const int q = blockIdx.x * G::LPB + l;
+  grid += slice_grid(a, blockIdx.y);
   C* line = buf + l * G::LS;
   C x[16];
 #pragma unroll
@@ -63,7 +69,7 @@ __global__ __launch_bounds__((LineGeo<R, L>::NT)) void k_fft_x_fwd(FArgs a, cons
   if (q < nlines) {
     const int iy = q % N1, iz = q / N1;
     const double fr = line_factor(a, iy, iz, true);
-    const C* src = f + (size_t)q * N0 * a.ist;
+    const C* src = f + slice_off(a.s0 + (int)blockIdx.y, a.Bsl, a.P) + (size_t)q * N0 * a.ist;
     double fc[16];
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
@@ -105,6 +111,7 @@ __global__ __launch_bounds__((LineGeo<R, L>::NT)) void k_fft_x_adj(FArgs a, cons
   const int nlines = a.N[1] * a.N[2];
   const int l = threadIdx.x / G::TL, j0 = threadIdx.x % G::TL;
   const int q = blockIdx.x * G::LPB + l;
+  grid += slice_grid(a, blockIdx.y);
   C* line = buf + l * G::LS;
   C x[16];
 #pragma unroll
@@ -120,7 +127,7 @@ __global__ __launch_bounds__((LineGeo<R, L>::NT)) void k_fft_x_adj(FArgs a, cons
   if (q < nlines) {
     const int iy = q % N1, iz = q / N1;
     const double fr = line_factor(a, iy, iz, false) * a.oscale;
-    C* dst = f + (size_t)q * N0 * a.ist;
+    C* dst = f + slice_off(a.s0 + (int)blockIdx.y, a.Bsl, a.P) + (size_t)q * N0 * a.ist;
 #pragma unroll
     for (int k = 0; k < 16; ++k) {
       const int ix = image_idx(j0 + k * G::TL, N0, L, Na0);
@@ -150,7 +157,7 @@ __global__ __launch_bounds__((LineGeo<R, L>::NT)) void k_fft_col(FArgs a, typena
   const int c = blockIdx.y;
   const int gc = call ? c : grid_pos(c, a.N[o], a.L[o], a.Na[o]);
   const int x0 = blockIdx.x * G::LPB;
-  const size_t base = (size_t)gc * a.gstr[o] + x0;
+  const size_t base = slice_grid(a, blockIdx.z) + (size_t)gc * a.gstr[o] + x0;
   const long long st = a.gstr[d];
   const int Nd = a.N[d], Nad = a.Na[d];
   const int xl = threadIdx.x % G::LPB, j0 = threadIdx.x / G::LPB;
@@ -175,7 +182,7 @@ hipError_t x_pass(bool fwd, const FArgs& a, hipStream_t s, const void* in, void*
   using C = typename cpx<R>::T;
   const int nlines = a.N[1] * a.N[2];
   using G = LineGeo<R, L>;
-  const dim3 g((unsigned)((nlines + G::LPB - 1) / G::LPB)), b(G::NT);
+  const dim3 g((unsigned)((nlines + G::LPB - 1) / G::LPB), (unsigned)a.nsl), b(G::NT);
   if (fwd) hipLaunchKernelGGL((k_fft_x_fwd<R, L>), g, b, 0, s, a, (const C*)in, (C*)out);
   else hipLaunchKernelGGL((k_fft_x_adj<R, L>), g, b, 0, s, a, (const C*)in, (C*)out);
   return hipGetLastError();
@@ -189,7 +196,7 @@ hipError_t col_pass(bool fwd, const FArgs& a, hipStream_t s, void* grid, int d) 
   const int call = d == 2 ? 1 : 0;
   const int nc = call ? a.L[o] : a.N[o];
   using G = LineGeo<R, L>;
-  const dim3 g((unsigned)((a.L[0] + G::LPB - 1) / G::LPB), (unsigned)nc), b(G::NT);
+  const dim3 g((unsigned)((a.L[0] + G::LPB - 1) / G::LPB), (unsigned)nc, (unsigned)a.nsl), b(G::NT);
   if (fwd) hipLaunchKernelGGL((k_fft_col<R, L, false, 1>), g, b, 0, s, a, (C*)grid, d, call);
   else hipLaunchKernelGGL((k_fft_col<R, L, true, 2>), g, b, 0, s, a, (C*)grid, d, call);
   return hipGetLastError();

@@ -506,8 +506,11 @@ hipError_t launch_inv_perm(const int* perm, int* iperm, long long n, hipStream_t
 template <typename C>
 __global__ __launch_bounds__(256) void k_gather_nodes(const C* __restrict__ in, long long is,
                                                       const int* __restrict__ idx, C* __restrict__ out,
-                                                      long long os, long long n) {
+                                                      long long os, long long n, int s0) {
   constexpr int U = 4;
+  // blockIdx.y: slice s0 + blockIdx.y of a directional plan (os slices side by side)
+  in += (size_t)blockIdx.y * n;
+  out += slice_off(s0 + (int)blockIdx.y, os, n);
   const long long b = (long long)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   for (long long i0 = b * 256 * U + threadIdx.x; i0 < n; i0 += (long long)gridDim.x * 256 * U) {
     int j[U];
@@ -523,15 +526,15 @@ __global__ __launch_bounds__(256) void k_gather_nodes(const C* __restrict__ in, 
 }
 
 hipError_t launch_gather_nodes(bool dbl, const void* in, long long is, const int* idx, void* out, long long os,
-                               long long n, hipStream_t s) {
+                               long long n, hipStream_t s, int s0, int nsl) {
   if (n <= 0) return hipSuccess;
   const unsigned blocks = (unsigned)(8 * ((std::min<long long>((n + 1023) / 1024, 65536) + 7) / 8));
   if (dbl)
-    hipLaunchKernelGGL(k_gather_nodes<double2>, dim3(blocks), dim3(256), 0, s, (const double2*)in, is, idx,
-                       (double2*)out, os, n);
+    hipLaunchKernelGGL(k_gather_nodes<double2>, dim3(blocks, nsl), dim3(256), 0, s, (const double2*)in, is, idx,
+                       (double2*)out, os, n, s0);
   else
-    hipLaunchKernelGGL(k_gather_nodes<float2>, dim3(blocks), dim3(256), 0, s, (const float2*)in, is, idx,
-                       (float2*)out, os, n);
+    hipLaunchKernelGGL(k_gather_nodes<float2>, dim3(blocks, nsl), dim3(256), 0, s, (const float2*)in, is, idx,
+                       (float2*)out, os, n, s0);
   return hipGetLastError();
 }
 
@@ -546,7 +549,7 @@ hipError_t launch_fold(int D, bool dbl, int W, const KArgs& a, hipStream_t s, vo
   if (D == 3) return launch_fold_d3(dbl, W, a, s, grid);
   long long rows = 1;
   for (int d = 1; d < D; ++d) rows *= a.Nt[d];
-  const dim3 g((a.Nt[0] + 255) / 256, (unsigned)std::min<long long>(rows, 65535)), blk(256);
+  const dim3 g((a.Nt[0] + 255) / 256, (unsigned)std::min<long long>(rows, 65535), a.nsl), blk(256);
 #define NFFTM_FOLD(DD)                                                                   \
   if (D == DD) {                                                                         \
     if (dbl) hipLaunchKernelGGL((k_fold<double, DD>), g, blk, 0, s, a, (double2*)grid);  \

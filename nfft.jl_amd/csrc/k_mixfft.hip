@@ -278,8 +278,7 @@ __device__ __forceinline__ int mix_id(int total) {
 }
 
 __device__ __forceinline__ size_t slice_start(const MixArgs& a) {
-  const long long s = a.s0 + (long long)blockIdx.y;
-  return (size_t)(s % a.Bsl + s / a.Bsl * a.Bsl * a.P);
+  return (size_t)slice_off(a.s0 + (int)blockIdx.y, a.Bsl, a.P);
 }
 __device__ __forceinline__ size_t slice_grid(const MixArgs& a) {
   return (size_t)(a.nsl - 1 - (int)blockIdx.y) * (size_t)a.Q;

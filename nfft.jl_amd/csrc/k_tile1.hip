@@ -99,6 +99,7 @@ __global__ __launch_bounds__(NT1) void k_interp1p(KArgs a, const typename cpx<R>
   const int4 it = a.items[item];
   C* tile = (C*)smem;
   const int t0 = it.x * a.T[0];
+  grid += slice_slot(a, blockIdx.y);
   // the first node's coordinate and index load during the staging, each
   // later node's during the one before
   int j = it.y + (int)threadIdx.x;
@@ -127,8 +128,8 @@ __global__ __launch_bounds__(NT1) void k_interp1p(KArgs a, const typename cpx<R>
       ar = fma(w[l], v.x, ar);
       ai = fma(w[l], v.y, ai);
     }
-    if (a.fsort) ((C*)a.fsort)[j] = C{ar * osc, ai * osc};
-    else fhat[(long long)pj * a.fst] = C{ar * osc, ai * osc};
+    if (a.fsort) ((C*)a.fsort)[(size_t)blockIdx.y * a.M + j] = C{ar * osc, ai * osc};
+    else fhat[slice_nodes(a, blockIdx.y) + (long long)pj * a.fst] = C{ar * osc, ai * osc};
   }
 }
 
@@ -142,6 +143,7 @@ __global__ __launch_bounds__(NT1) void k_spread1p(KArgs a, const typename cpx<R>
   double* acc = (double*)smem;  // re plane [0, te), im plane [te, 2 te)
   const int te = a.tileElems;
   const int t0 = it.x * a.T[0];
+  fhat += slice_nodes(a, blockIdx.y);
   // node coordinate and value one node ahead
   int j = it.y + (int)threadIdx.x;
   double kn = 0;
@@ -170,7 +172,7 @@ __global__ __launch_bounds__(NT1) void k_spread1p(KArgs a, const typename cpx<R>
     }
   }
   __syncthreads();
-  C* out = (C*)a.scratch + (size_t)item * a.padCells;
+  C* out = (C*)a.scratch + slice_scratch(a, blockIdx.y) + (size_t)item * a.padCells;
   for (int i = threadIdx.x; i < a.padCells; i += NT1) out[i] = C{(R)acc[i], (R)acc[te + i]};
 }
 
@@ -183,13 +185,13 @@ static hipError_t poly1_go(bool spread, const KArgs& a, hipStream_t s, const voi
     auto k = k_spread1p<R, W>;
     if (hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
       return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL(k, dim3(nblk), dim3(NT1), lds, s, a, (const C*)in);
+    hipLaunchKernelGGL(k, dim3(nblk, a.nsl), dim3(NT1), lds, s, a, (const C*)in);
   } else {
     const size_t lds = (size_t)a.padCells * sizeof(C);
     auto k = k_interp1p<R, W>;
     if (hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
       return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL(k, dim3(nblk), dim3(NT1), lds, s, a, (const C*)in, (C*)out);
+    hipLaunchKernelGGL(k, dim3(nblk, a.nsl), dim3(NT1), lds, s, a, (const C*)in, (C*)out);
   }
   return hipGetLastError();
 }

@@ -119,8 +119,29 @@ struct KArgs {
   void* scratch;       // nitems padded tiles (dense, px fastest)
   const int* tstart;   // items of tile t: [tstart[t], tstart[t+1])
   int ntile_all;       // product of ntiles
-  int maxcand;         // covering (tile, offset) pairs per dim (fold)
+  // slices s0 .. s0 + nsl - 1 of a directional plan in one launch (1-D and 2-D
+  // tile kernels and their fold; otherwise s0 = 0, nsl = 1): the node values
+  // of slice s start at element s % Bsl + (s / Bsl) Bsl M, its grid is slot
+  // nsl - 1 - (s - s0) of consecutive grids of Q points (the last slice in
+  // slot 0, the plan's grid), its scratch slots follow those of s - 1
+  int s0, nsl;
+  long long Bsl, Q;
 };
+
+// (Bsl < 2^31; slice 0, the only one of an ordinary plan, needs no division)
+__host__ __device__ __forceinline__ long long slice_off(int s, long long Bsl, long long len) {
+  if (s == 0) return 0;
+  const unsigned q = (unsigned)s / (unsigned)Bsl;
+  return (long long)((unsigned)s - q * (unsigned)Bsl) + (long long)q * Bsl * len;
+}
+// i = the launch's slice index (a block index)
+__device__ __forceinline__ long long slice_nodes(const KArgs& a, int i) { return slice_off(a.s0 + i, a.Bsl, a.M); }
+__device__ __forceinline__ size_t slice_slot(const KArgs& a, int i) {
+  return (size_t)(a.nsl - 1 - i) * (size_t)a.Q;
+}
+__device__ __forceinline__ size_t slice_scratch(const KArgs& a, int i) {
+  return (size_t)i * (size_t)a.nitems * (size_t)a.padCells;
+}
 
 // k * Ntilde rounded to FP64 before any further use, as the reference
 // computes kscale (src/precomputation.jl:538): kept out of a fused multiply-add
@@ -595,7 +616,8 @@ __global__ __launch_bounds__(NT) void k_spread_tile(KArgs a, const typename cpx<
   // XCD (xcd_item) leave the XCDs unevenly loaded
   const int item = blockIdx.x;
   if (item >= a.nitems) return;
-  spread_tile_item<R, D, W, NT>(a, item, fhat, (typename cpx<R>::T*)a.scratch);
+  spread_tile_item<R, D, W, NT>(a, item, fhat + slice_nodes(a, blockIdx.y),
+                                (typename cpx<R>::T*)a.scratch + slice_scratch(a, blockIdx.y));
 }
 
 // Fold: grid point x sums, over the padded tiles covering it, the scratch
@@ -662,7 +684,8 @@ __device__ __forceinline__ typename cpx<R>::T fold_sum(const KArgs& a, const typ
 template <typename R, int D>
 __global__ __launch_bounds__(256) void k_fold(KArgs a, typename cpx<R>::T* __restrict__ grid) {
   using C = typename cpx<R>::T;
-  const C* scr = (const C*)a.scratch;
+  const C* scr = (const C*)a.scratch + slice_scratch(a, blockIdx.z);
+  grid += slice_slot(a, blockIdx.z);
   const int x = blockIdx.x * 256 + threadIdx.x;
   const int ny = D >= 2 ? a.Nt[1] : 1;
   const int nrows = (D >= 2 ? a.Nt[1] : 1) * (D == 3 ? a.Nt[2] : 1);
@@ -756,7 +779,7 @@ __global__ __launch_bounds__(NT) void k_interp_tile(KArgs a, const typename cpx<
                                                     typename cpx<R>::T* __restrict__ fhat) {
   const int item = blockIdx.x;  // round robin over the XCDs (k_spread_tile)
   if (item >= a.nitems) return;
-  interp_tile_item<R, D, W, NT>(a, item, grid, fhat);
+  interp_tile_item<R, D, W, NT>(a, item, grid + slice_slot(a, blockIdx.y), fhat + slice_nodes(a, blockIdx.y));
 }
 
 }  // namespace nfftm

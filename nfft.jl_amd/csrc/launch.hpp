@@ -33,6 +33,8 @@ struct FArgs {
   const double* fac[3];
   const void* tw[3];
   double oscale;
+  int s0, nsl;  // slices of one launch (KArgs), images of P and grids of Q points
+  long long Bsl, P, Q;
 };
 
 // Power-of-two grids within the line kernels' LDS (FP32: 16..2048 points
@@ -77,8 +79,10 @@ hipError_t launch_shift_sign(bool dbl, void* x, const ToepArgs& a, hipStream_t s
 // iperm[perm[j]] = j, and out[i * os] = in[idx[i] * is] (node values between
 // the caller's and the sorted order).
 hipError_t launch_inv_perm(const int* perm, int* iperm, long long n, hipStream_t s);
+// nsl slices s0 .. of a directional plan: their sorted values follow one
+// another, their outputs start at slice_off(s, os, n).
 hipError_t launch_gather_nodes(bool dbl, const void* in, long long is, const int* idx, void* out, long long os,
-                               long long n, hipStream_t s);
+                               long long n, hipStream_t s, int s0, int nsl);
 
 // LDS bytes of a tile kernel.
 size_t tile_lds_bytes(int D, bool dbl, int W, int tileElems);

@@ -419,6 +419,9 @@ struct nfftm_plan_s {
   // arguments: Bsl while a directional transform runs, 1 otherwise (the
   // plan's own work vectors are contiguous)
   i64 io_stride = 1;
+  // slices of the running launches (1 outside a directional transform), and
+  // how many of them d_grid and d_scratch hold
+  int sl0 = 0, sln = 1, gcap = 1, scap = 1;
   // 3-D scratch slots in halo/interior block layout: halos (m - 1, m cells)
   // no wider than any tile, a partial last one included
   bool blocked3() const {
@@ -616,6 +619,10 @@ struct nfftm_plan_s {
     a.tstart = d_tstart.p;
     a.ntile_all = ntiles[0] * ntiles[1] * ntiles[2];
     a.fst = io_stride;
+    a.s0 = sl0;
+    a.nsl = sln;
+    a.Bsl = io_stride;
+    a.Q = Q;
     return a;
   }
 
@@ -638,6 +645,11 @@ struct nfftm_plan_s {
     }
     a.oscale = 1.0;
     a.ist = io_stride;
+    a.s0 = sl0;
+    a.nsl = sln;
+    a.Bsl = io_stride;
+    a.P = P;
+    a.Q = Q;
     return a;
   }
 
@@ -663,7 +675,7 @@ struct nfftm_plan_s {
     a.st = gs[d];
     if (d == 0) {
       a.nlines = (int)(n[1] * n[2]);
-      a.lpb = mix_shape(dbl(), false, a.ln, a.nlines, 1);
+      a.lpb = mix_shape(dbl(), false, a.ln, a.nlines, sln);
       a.total = (a.nlines + a.lpb - 1) / a.lpb;
     } else {
       const int o = 3 - d;
@@ -674,7 +686,7 @@ struct nfftm_plan_s {
       a.ost = gs[o];
       a.nx = (int)l[0];
       const i64 outer = a.oall ? l[o] : n[o];
-      a.lpb = mix_shape(dbl(), true, a.ln, a.nx, outer);
+      a.lpb = mix_shape(dbl(), true, a.ln, a.nx, outer * sln);
       a.nchunk = (a.nx + a.lpb - 1) / a.lpb;
       a.total = (int)(a.nchunk * outer);
     }
@@ -691,8 +703,9 @@ struct nfftm_plan_s {
     a.st2 = gs[2];
     a.oscale = 1.0;
     a.ist = io_stride;
-    a.nsl = 1;
-    a.Bsl = 1;
+    a.s0 = sl0;
+    a.nsl = sln;
+    a.Bsl = io_stride;
     a.P = P;
     a.Q = Q;
     return a;
@@ -903,6 +916,28 @@ int build_records(nfftm_plan_s& p) {
   return NFFTM_OK;
 }
 
+// Directional plans on the 1-D and 2-D tile kernels run several slices per
+// launch: as many grids as fit 512 MiB and as many scratch areas as fit
+// another 512 MiB, at most 256 of each (one slice of a 480^2 grid takes about
+// 9 us of launches and latency per kernel, eight kernels; 32 of them together
+// fill the GPU).  The 3-D kernels and the three-pass 1-D FFT fill it with one.
+constexpr size_t SLICE_BYTES = (size_t)512 << 20;
+int slice_cap(const nfftm_plan_s& p, size_t bytes) {
+  if (!p.dir() || !p.tiled || p.D == 3 || p.f1 || p.Bsl > 0x7fffffff || p.Asl > 0x7fffffff / p.Bsl) return 1;
+  return (int)std::max<i64>(1, std::min<i64>({p.Bsl * p.Asl, 256, (i64)(SLICE_BYTES / std::max<size_t>(1, bytes))}));
+}
+int alloc_grid(nfftm_plan_s& p) {
+  p.gcap = slice_cap(p, (size_t)p.Q * p.celem());
+  HIPCHK(p.d_grid.alloc((size_t)p.gcap * p.Q * p.celem()));
+  return NFFTM_OK;
+}
+int alloc_scratch(nfftm_plan_s& p) {
+  const size_t one = std::max<size_t>(1, (size_t)p.nitems) * p.slot_cells() * p.celem();
+  p.scap = slice_cap(p, one);
+  HIPCHK(p.d_scratch.alloc((size_t)p.scap * one));
+  return NFFTM_OK;
+}
+
 // sort, split each tile's nodes into work items, gather the shifted nodes in
 // tile order.
 int set_nodes(nfftm_plan_s& p, const double* k, i64 M) {
@@ -996,7 +1031,7 @@ int set_nodes(nfftm_plan_s& p, const double* k, i64 M) {
     HIPCHK(launch_sparse_build(p.dbl(), p.W, p.kargs(), p.stream, p.d_bcols.p, p.d_bvals.p));
   }
   if (p.tiled) {
-    HIPCHK(p.d_scratch.alloc(std::max<size_t>(1, (size_t)nitems) * p.slot_cells() * p.celem()));
+    if (int rc = alloc_scratch(p)) return rc;
     // node records in tile order, built on the device (1-D polynomial-window
     // plans evaluate the window in their kernels; a batch that takes such a
     // plan builds its records then)
@@ -1005,7 +1040,7 @@ int set_nodes(nfftm_plan_s& p, const double* k, i64 M) {
     p.d_iperm.reset();
     p.d_fsort.reset();
     if (p.sorted_io() && M > 0) {
-      HIPCHK(p.d_fsort.alloc((size_t)M * p.celem()));
+      HIPCHK(p.d_fsort.alloc((size_t)p.scap * M * p.celem()));
       HIPCHK(p.d_iperm.alloc((size_t)M));
       HIPCHK(launch_inv_perm(p.d_perm.p, p.d_iperm.p, M, p.stream));
     }
@@ -1107,7 +1142,7 @@ int run_conv(nfftm_plan_s& p, bool spread, const void* in, void* out, bool stand
       // caller's order
       a.fsort = p.d_fsort.p;
       e = launch_tile(p.D, false, p.dbl(), p.W, p.NT, a, p.lds, p.stream, in, nullptr);
-      if (e == hipSuccess) e = launch_gather_nodes(p.dbl(), p.d_fsort.p, 1, p.d_iperm.p, out, a.fst, p.M, p.stream);
+      if (e == hipSuccess) e = launch_gather_nodes(p.dbl(), p.d_fsort.p, 1, p.d_iperm.p, out, a.fst, p.M, p.stream, p.sl0, p.sln);
     } else if (p.tiled)
       e = launch_tile(p.D, spread, p.dbl(), p.W, p.NT, a, p.lds, p.stream, in, spread ? nullptr : out);
     else if (p.sparse)
@@ -1187,6 +1222,14 @@ int typed_conv(nfftm_plan_s& p, bool spread, const void* in, int tin, i64 nin, v
   return NFFTM_OK;
 }
 
+// Image and grid of slice i of the running launches (KArgs).
+const void* slice_image(const nfftm_plan_s& p, const void* f, int i) {
+  return (const char*)f + (size_t)slice_off(p.sl0 + i, p.io_stride, p.P) * p.celem();
+}
+void* slice_grid(const nfftm_plan_s& p, int i) {
+  return p.d_grid.p + (size_t)(p.sln - 1 - i) * (size_t)p.Q * p.celem();
+}
+
 // Forward deconvolution and FFT into the grid: stage 0 (deconvolve!, or the
 // pruned dimension-1 pass with the deconvolution fused) and stage 1 (the FFT,
 // or the remaining pruned passes), with an optional timer mark in between.
@@ -1224,10 +1267,13 @@ int forward_to_grid(nfftm_plan_s& p, const void* f, Mark&& mark) {
     HIPCHK(launch_fft1_fwd(p.dbl(), a, p.stream, f, p.d_grid.p, 1));
     return NFFTM_OK;
   }
-  if (int rc = run_deconv(p, true, f, p.d_grid.p)) return rc;
+  for (int i = 0; i < p.sln; ++i)
+    if (int rc = run_deconv(p, true, slice_image(p, f, i), slice_grid(p, i))) return rc;
   if (int rc = mark()) return rc;
   ProfScope ps(p, 1);
-  return p.fft->exec(true, p.d_grid.p, p.celem(), p.stream);
+  for (int i = 0; i < p.sln; ++i)
+    if (int rc = p.fft->exec(true, slice_grid(p, i), p.celem(), p.stream)) return rc;
+  return NFFTM_OK;
 }
 
 // Adjoint inverse FFT of the grid and deconvolution into f: stage 5 and
@@ -1277,10 +1323,13 @@ int grid_to_image(nfftm_plan_s& p, void* f, Mark&& mark, bool fused = false) {
   }
   {
     ProfScope ps(p, 5);
-    if (int rc = p.fft->exec(false, p.d_grid.p, p.celem(), p.stream)) return rc;
+    for (int i = 0; i < p.sln; ++i)
+      if (int rc = p.fft->exec(false, slice_grid(p, i), p.celem(), p.stream)) return rc;
   }
   if (int rc = mark()) return rc;
-  return run_deconv(p, false, p.d_grid.p, f);
+  for (int i = 0; i < p.sln; ++i)
+    if (int rc = run_deconv(p, false, slice_grid(p, i), const_cast<void*>(slice_image(p, f, i)))) return rc;
+  return NFFTM_OK;
 }
 
 struct Timer {
@@ -1328,15 +1377,18 @@ int create_impl(nfftm_plan_s& p, const double* k) {
     choose_tiles(p);
     p.tiled = tiles_ok(p);
   }
-  if (int rc = build_tables(p)) return rc;
-  if (int rc = set_nodes(p, k, p.M)) return rc;
-  HIPCHK(p.d_grid.alloc((size_t)p.Q * p.celem()));
-  p.fft.reset(new FFTStage());
-  if (int rc = p.fft->build(p.D, p.Nt, p.dbl())) return rc;
+  // the FFT stage: pruned passes where they are built for the grid
   p.pfft = !(p.flags & NFFTM_FLAG_ROCFFT) && pruned_fft_supported(p.D, p.N, p.Nt, p.dbl());
   p.mix = !(p.flags & NFFTM_FLAG_ROCFFT) && !p.pfft && p.D <= 3 && p.Q < (1LL << 31);
   for (int d = 0; d < p.D && p.mix; ++d)
     p.mix = p.N[d] <= p.Nt[d] && mix_factor(p.Nt[d], p.dbl(), p.D == 1, &p.mixln[d]);
+  p.f1 = !p.pfft && !p.mix && p.D == 1 && !(p.flags & NFFTM_FLAG_ROCFFT) &&
+         fft1_factor(p.Nt[0], p.N[0], p.dbl(), &p.f1n1, &p.f1Lm);
+  if (int rc = build_tables(p)) return rc;
+  if (int rc = set_nodes(p, k, p.M)) return rc;
+  if (int rc = alloc_grid(p)) return rc;
+  p.fft.reset(new FFTStage());
+  if (int rc = p.fft->build(p.D, p.Nt, p.dbl())) return rc;
   if (p.pfft || p.mix) {
     // twiddle tables exp(-2 pi i k / Nt_d) as (cos, sin) of 2 pi k / Nt_d,
     // FP64 on the host, stored in the data precision
@@ -1365,8 +1417,6 @@ int create_impl(nfftm_plan_s& p, const double* k) {
     HIPCHK(p.d_tw.alloc(bytes));
     HIPCHK(hipMemcpy(p.d_tw.p, h.data(), bytes, hipMemcpyHostToDevice));
   }
-  p.f1 = !p.pfft && !p.mix && p.D == 1 && !(p.flags & NFFTM_FLAG_ROCFFT) &&
-         fft1_factor(p.Nt[0], p.N[0], p.dbl(), &p.f1n1, &p.f1Lm);
   if (p.f1) {
     // (cos, sin)(2 pi j / n1) and (2 pi j / Lm) in the data precision,
     // (2 pi (j << sh) / Nt) and (2 pi j / Nt), 2^sh >= sqrt(Nt), in FP64
@@ -1889,6 +1939,13 @@ int nfftm_plan_create_dims(nfftm_plan* out, int prec, int D, const int64_t* N, i
       if (d < dim_lo) p->Bsl *= N[d];
       if (d > dim_hi) p->Asl *= N[d];
     }
+    std::unique_ptr<nfftm_plan_s> own(p);
+    if (int rc = alloc_grid(*p)) return rc;
+    if (p->tiled) {
+      if (int rc = alloc_scratch(*p)) return rc;
+      if (p->d_fsort.p) HIPCHK(p->d_fsort.alloc((size_t)p->scap * p->M * p->celem()));
+    }
+    own.release();
   }
   *out = p;
   return NFFTM_OK;
@@ -1930,12 +1987,38 @@ int for_slices(nfftm_plan_s& p, const void* in, i64 in_len, void* out, i64 out_l
   return NFFTM_OK;
 }
 
+// fn(in, out) for the slices of a directional transform, several per launch
+// where the plan's buffers hold several grids: fn gets the caller's arrays and
+// the kernels find their slices (sl0, sln); the plan's grid is left with the
+// last slice's.  Otherwise as for_slices.
+template <typename F>
+int for_chunks(nfftm_plan_s& p, const void* in, i64 in_len, void* out, i64 out_len, F&& fn) {
+  const int cap = std::min(p.gcap, p.scap);
+  if (!p.dir() || cap == 1) return for_slices(p, in, in_len, out, out_len, fn);
+  struct Reset {
+    nfftm_plan_s& p;
+    ~Reset() {
+      p.io_stride = 1;
+      p.sl0 = 0;
+      p.sln = 1;
+    }
+  } reset{p};
+  p.io_stride = p.Bsl;
+  const i64 S = p.Bsl * p.Asl;
+  for (i64 s = 0; s < S; s += cap) {
+    p.sl0 = (int)s;
+    p.sln = (int)std::min<i64>(cap, S - s);
+    if (int rc = fn(in, out)) return rc;
+  }
+  return NFFTM_OK;
+}
+
 // Launch sequence of one direction on p.stream: forward = deconvolve, FFT,
 // interpolate; adjoint = spread (+ fold), backward FFT, deconvolve_transpose;
 // for every slice of a directional plan.
 int enqueue_transform(nfftm_plan_s& p, bool fwd, const void* in, void* out) {
   auto none = [] { return (int)NFFTM_OK; };
-  return for_slices(p, in, fwd ? p.P : p.M, out, fwd ? p.M : p.P, [&](const void* i, void* o) -> int {
+  return for_chunks(p, in, fwd ? p.P : p.M, out, fwd ? p.M : p.P, [&](const void* i, void* o) -> int {
     if (fwd) {
       if (int rc = forward_to_grid(p, i, none)) return rc;
       if (p.M) return run_conv(p, false, p.d_grid.p, o);
@@ -1999,7 +2082,7 @@ int nfftm_forward(nfftm_plan p, const void* f, void* fhat) {
     return graph_transform(*p, true, f, fhat);
   const bool acc = p->dir();
   if (acc) p->timing[1] = p->timing[2] = p->timing[3] = 0;
-  return for_slices(*p, f, p->P, fhat, p->M, [&](const void* fs, void* fhs) -> int {
+  return for_chunks(*p, f, p->P, fhat, p->M, [&](const void* fs, void* fhs) -> int {
     Timer t(*p);
     if (int rc = t.mark(0)) return rc;
     if (int rc = forward_to_grid(*p, fs, [&] { return t.mark(1); })) return rc;
@@ -2020,7 +2103,7 @@ int nfftm_adjoint(nfftm_plan p, const void* fhat, void* f) {
     return graph_transform(*p, false, fhat, f);
   const bool acc = p->dir();
   if (acc) p->timing[4] = p->timing[5] = p->timing[6] = 0;
-  return for_slices(*p, fhat, p->M, f, p->P, [&](const void* fhs, void* fs) -> int {
+  return for_chunks(*p, fhat, p->M, f, p->P, [&](const void* fhs, void* fs) -> int {
     Timer t(*p);
     if (int rc = t.mark(0)) return rc;
     const bool fused = fused_fold(*p);
