@@ -137,6 +137,10 @@ int nfftm_plan_create_dims(nfftm_plan* out, int prec, int D, const int64_t* N, i
 /* nodes!(p, k): src/implementation.jl:108-141 (AbstractNFFTs/src/interface.jl:211).
  * M may differ from the plan's current M. */
 int nfftm_nodes(nfftm_plan p, const double* k_host, int64_t M);
+/* The same for nodes held as D rows of M values, row r the coordinate of
+ * dimension D - r (1-based): a C-order array of shape (D, M) whose rows pair
+ * with the axes of a C-order image.  No transposed copy is made. */
+int nfftm_nodes_rows(nfftm_plan p, const double* k_host, int64_t M);
 
 /* mul!(fHat, p, f): src/implementation.jl:155-172 (interface.jl:170).
  * f: prod(N) complex, fhat: M complex. */

@@ -30,24 +30,31 @@ __device__ __forceinline__ double shifted(double x) {
   return x;
 }
 
-// Tile of node j (k in the caller's layout, D values per node).
-__device__ __forceinline__ int node_tile(const BinArgs& a, const double* __restrict__ k, long long j) {
-  long long t = 0, str = 1;
+// Tile of node j (k in the caller's layout).  A coordinate outside
+// [-1/2, 1/2] (or NaN) is flagged and taken as 0: the host reads the flag
+// before anything of the plan changes.
+__device__ __forceinline__ int node_tile(const BinArgs& a, const double* __restrict__ k, long long j, int* bad) {
+  int t = 0, str = 1;
   for (int d = 0; d < a.D; ++d) {
-    const double kscale = shifted(k[d + (long long)a.D * j]) * (double)a.Nt[d];
-    long long c = (long long)kscale;
+    double x = k[d * a.sd + j * a.sj];
+    if (!(fabs(x) <= 0.5)) {
+      *bad = 1;
+      x = 0;
+    }
+    const double kscale = shifted(x) * (double)a.Nt[d];
+    int c = (int)kscale;
     if (c >= a.Nt[d]) c -= a.Nt[d];
-    t += (c / a.T[d]) * str;
+    t += (int)((unsigned)c / (unsigned)a.T[d]) * str;
     str *= a.ntiles[d];
   }
-  return (int)t;
+  return t;
 }
 
 __global__ __launch_bounds__(BT) void k_bin_keys(BinArgs a, const double* __restrict__ k, int* __restrict__ key,
                                                  int* __restrict__ idx, int* __restrict__ cnt) {
   const long long j = (long long)blockIdx.x * BT + threadIdx.x;
   if (j >= a.M) return;
-  const int t = node_tile(a, k, j);
+  const int t = node_tile(a, k, j, &cnt[a.ntile]);
   key[j] = t;
   idx[j] = (int)j;
   atomicAdd(&cnt[t], 1);
@@ -64,7 +71,7 @@ __global__ __launch_bounds__(BT) void k_bin_keys_lds(BinArgs a, const double* __
   for (int i = threadIdx.x; i < a.ntile; i += BT) hist[i] = 0;
   __syncthreads();
   for (long long j = (long long)blockIdx.x * BT + threadIdx.x; j < a.M; j += (long long)gridDim.x * BT) {
-    const int t = node_tile(a, k, j);
+    const int t = node_tile(a, k, j, &cnt[a.ntile]);
     key[j] = t;
     idx[j] = (int)j;
     atomicAdd(&hist[t], 1);
@@ -77,51 +84,53 @@ __global__ __launch_bounds__(BT) void k_bin_keys_lds(BinArgs a, const double* __
 // One workgroup: off = exclusive scan of cnt (ntile + 1 entries), ioff =
 // exclusive scan of ceil(cnt / CH) (work items per tile); stats[0] = number
 // of work items, stats[1] = tiles of more than one, stats[2] = 0 (the counter
-// of k_bin_items).
+// of k_bin_items), stats[3] = the bad-node flag cnt[ntile].  Each thread sums
+// its run of tiles, the 1024 sums are scanned by wavefront shuffles (by one
+// thread they took 20 of 27 us).
 constexpr int ST = 1024;
+__device__ __forceinline__ int3 wave_scan(int3 v) {  // inclusive
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int x = __shfl_up(v.x, o), y = __shfl_up(v.y, o), z = __shfl_up(v.z, o);
+    if ((int)(threadIdx.x & 63) >= o) v.x += x, v.y += y, v.z += z;
+  }
+  return v;
+}
 __global__ __launch_bounds__(ST) void k_bin_scan(BinArgs a, const int* __restrict__ cnt, int* __restrict__ off,
                                                  int* __restrict__ ioff, int* __restrict__ stats) {
-  __shared__ long long s_n[ST], s_i[ST];
-  __shared__ int s_mul[ST];
+  __shared__ int3 s_wave[ST / 64];
   const int n = a.ntile;
   const int per = (n + ST - 1) / ST;
-  const int b = threadIdx.x * per, e = min(n, b + per);
-  long long sn = 0, si = 0;
-  int mx = 0;  // tiles of several items
+  const int b = min(n, (int)threadIdx.x * per), e = min(n, b + per);
+  int3 s{0, 0, 0};  // nodes, items, tiles of several items
   for (int t = b; t < e; ++t) {
     const int c = cnt[t];
     const int it = (c + a.CH - 1) / a.CH;
-    sn += c;
-    si += it;
-    mx += it > 1;
+    s.x += c;
+    s.y += it;
+    s.z += it > 1;
   }
-  s_n[threadIdx.x] = sn;
-  s_i[threadIdx.x] = si;
-  s_mul[threadIdx.x] = mx;
+  int3 inc = wave_scan(s);
+  if ((threadIdx.x & 63) == 63) s_wave[threadIdx.x >> 6] = inc;
   __syncthreads();
-  if (threadIdx.x == 0) {  // ST partial sums: serial exclusive scan
-    long long an = 0, ai = 0;
-    int am = 0;
-    for (int w = 0; w < ST; ++w) {
-      const long long tn = s_n[w], ti = s_i[w];
-      s_n[w] = an;
-      s_i[w] = ai;
-      an += tn;
-      ai += ti;
-      am += s_mul[w];
-    }
-    off[n] = (int)an;
-    ioff[n] = (int)ai;
-    stats[0] = (int)ai;
-    stats[1] = am;
+  for (int w = 0; w < (int)(threadIdx.x >> 6); ++w) {
+    inc.x += s_wave[w].x;
+    inc.y += s_wave[w].y;
+    inc.z += s_wave[w].z;
+  }
+  if (threadIdx.x == ST - 1) {
+    off[n] = inc.x;
+    ioff[n] = inc.y;
+    stats[0] = inc.y;
+    stats[1] = inc.z;
     stats[2] = 0;
+    stats[3] = cnt[n];
   }
-  __syncthreads();
-  long long an = s_n[threadIdx.x], ai = s_i[threadIdx.x];
+  int an = inc.x - s.x, ai = inc.y - s.y;
   for (int t = b; t < e; ++t) {
     const int c = cnt[t];
-    off[t] = (int)an;
-    ioff[t] = (int)ai;
+    off[t] = an;
+    ioff[t] = ai;
     an += c;
     ai += (c + a.CH - 1) / a.CH;
   }
@@ -149,7 +158,13 @@ __global__ __launch_bounds__(BT) void k_bin_ks(BinArgs a, const double* __restri
   const long long s = (long long)blockIdx.x * BT + threadIdx.x;
   if (s >= a.M) return;
   const long long j = perm ? perm[s] : s;
-  for (int d = 0; d < a.D; ++d) ks[(long long)d * a.M + s] = shifted(k[d + (long long)a.D * j]);
+  for (int d = 0; d < a.D; ++d) ks[(long long)d * a.M + s] = shifted(k[d * a.sd + j * a.sj]);
+}
+
+// flag[0] = 1 if some coordinate is outside [-1/2, 1/2] or NaN.
+__global__ __launch_bounds__(BT) void k_check(const double* __restrict__ k, long long n, int* __restrict__ flag) {
+  const long long i = (long long)blockIdx.x * BT + threadIdx.x;
+  if (i < n && !(fabs(k[i]) <= 0.5)) flag[0] = 1;
 }
 
 __global__ __launch_bounds__(BT) void k_iota(int* __restrict__ p, long long n) {
@@ -161,9 +176,14 @@ inline unsigned blocks(long long n) { return (unsigned)((n + BT - 1) / BT); }
 
 }  // namespace
 
+// The radix passes for every M: up to 2^20 nodes rocPRIM would take its merge
+// sort, 17 launches and 91 us for 2 10^5 nodes.
+using SortConfig =
+    rocprim::radix_sort_config<rocprim::default_config, rocprim::default_config, rocprim::default_config, 0>;
+
 size_t bin_sort_temp_bytes(long long M, int key_bits) {
   size_t bytes = 0;
-  if (rocprim::radix_sort_pairs(nullptr, bytes, (int*)nullptr, (int*)nullptr, (int*)nullptr, (int*)nullptr,
+  if (rocprim::radix_sort_pairs<SortConfig>(nullptr, bytes, (int*)nullptr, (int*)nullptr, (int*)nullptr, (int*)nullptr,
                                 (size_t)M, 0, key_bits) != hipSuccess)
     return 0;
   return std::max<size_t>(bytes, 16);
@@ -184,7 +204,7 @@ hipError_t launch_bin_keys(const BinArgs& a, const double* k, int* key, int* idx
 hipError_t launch_bin_sort(const BinArgs& a, void* temp, size_t temp_bytes, int* key_in, int* key_out, int* idx_in,
                            int* idx_out, hipStream_t s) {
   if (a.M == 0) return hipSuccess;
-  return rocprim::radix_sort_pairs(temp, temp_bytes, key_in, key_out, idx_in, idx_out, (size_t)a.M, 0, a.key_bits,
+  return rocprim::radix_sort_pairs<SortConfig>(temp, temp_bytes, key_in, key_out, idx_in, idx_out, (size_t)a.M, 0, a.key_bits,
                                    s);
 }
 
@@ -203,6 +223,13 @@ hipError_t launch_bin_items(const BinArgs& a, const int* off, const int* ioff, i
 hipError_t launch_bin_ks(const BinArgs& a, const double* k, const int* perm, double* ks, hipStream_t s) {
   if (a.M == 0) return hipSuccess;
   hipLaunchKernelGGL(k_bin_ks, dim3(blocks(a.M)), dim3(BT), 0, s, a, k, perm, ks);
+  return hipGetLastError();
+}
+
+hipError_t launch_check_nodes(const double* k, long long n, int* flag, hipStream_t s) {
+  const hipError_t e = launch_fill0(flag, sizeof(int), s);
+  if (e != hipSuccess || n == 0) return e;
+  hipLaunchKernelGGL(k_check, dim3(blocks(n)), dim3(BT), 0, s, k, n, flag);
   return hipGetLastError();
 }
 

@@ -419,7 +419,7 @@ hipError_t launch_deconv_t_batch(bool dbl, int nblk, hipStream_t s, const DArgs*
 
 template <typename R, int D>
 static hipError_t records_w(int W, const KArgs& a, char* rec, hipStream_t s) {
-  const dim3 g((unsigned)a.nitems), b(256);
+  const dim3 g((unsigned)((a.M + 255) / 256)), b(256);
   switch (W) {
 #define NFFTM_REC(WW) \
   case WW:            \
@@ -434,7 +434,7 @@ static hipError_t records_w(int W, const KArgs& a, char* rec, hipStream_t s) {
 }
 
 hipError_t launch_node_records(int D, bool dbl, int W, const KArgs& a, void* rec, hipStream_t s) {
-  if (a.nitems == 0) return hipSuccess;
+  if (a.M == 0) return hipSuccess;
   char* r = (char*)rec;
   if (D == 1) return dbl ? records_w<double, 1>(W, a, r, s) : records_w<float, 1>(W, a, r, s);
   if (D == 2) return dbl ? records_w<double, 2>(W, a, r, s) : records_w<float, 2>(W, a, r, s);

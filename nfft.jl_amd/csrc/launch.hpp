@@ -124,9 +124,10 @@ hipError_t launch_deconv_t_batch(bool dbl, int nblk, hipStream_t s, const DArgs*
 // Node binning on the device (k_bin.hip).  Tiles per dimension as the tile
 // kernels use them; CH = most nodes of one work item; key_bits covers the
 // tile indices (ntile <= 2^key_bits).
+// Coordinate d of the caller's node j is k[d sd + j sj].
 struct BinArgs {
   int D;
-  long long M;
+  long long M, sd, sj;
   int Nt[3], T[3], ntiles[3];
   int ntile, CH, key_bits;
 };
@@ -138,6 +139,7 @@ hipError_t launch_bin_scan(const BinArgs& a, const int* cnt, int* off, int* ioff
 hipError_t launch_bin_items(const BinArgs& a, const int* off, const int* ioff, int4* items, int* tstart, int* multi,
                             int* nmulti, hipStream_t s);
 hipError_t launch_bin_ks(const BinArgs& a, const double* k, const int* perm, double* ks, hipStream_t s);
+hipError_t launch_check_nodes(const double* k, long long n, int* flag, hipStream_t s);
 hipError_t launch_iota(int* p, long long n, hipStream_t s);
 
 // Node records (weights, local cell, caller index) of every work item.

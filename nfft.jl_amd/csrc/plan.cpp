@@ -393,6 +393,16 @@ struct DevBuf {
     if (e == hipSuccess) n = count;
     return e;
   }
+  // room for count elements: what is there is kept (not its contents) unless
+  // it is too small or more than four times too large
+  hipError_t ensure(size_t count) {
+    if (n >= count && n <= 4 * count + 65536) return hipSuccess;
+    return alloc(count);
+  }
+  void swap(DevBuf& o) {
+    std::swap(p, o.p);
+    std::swap(n, o.n);
+  }
 };
 
 }  // namespace
@@ -500,7 +510,26 @@ struct nfftm_plan_s {
   double prof_ms[8] = {0};
   int64_t prof_cnt[8] = {0};
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
-  std::vector<double> k;  // caller's nodes (D x M), kept for copy()
+  // the caller's nodes on the device (Julia D x M, or krows: rows of M in
+  // reversed dimension order), for copy() and for binning them again
+  DevBuf<double> d_k;
+  bool krows = false;
+  // binning work arrays, kept from the first nodes! on
+  struct BinWork {
+    DevBuf<double> k;
+    DevBuf<int> key_in, key_out, idx_in, cnt, off, ioff, stats;
+    DevBuf<char> tmp;
+    int* h_stats = nullptr;  // pinned copy of stats
+    void release() {
+      k.reset();
+      for (auto* b : {&key_in, &key_out, &idx_in, &cnt, &off, &ioff, &stats}) b->reset();
+      tmp.reset();
+      if (h_stats) (void)hipHostFree(h_stats);
+      h_stats = nullptr;
+    }
+    ~BinWork() { release(); }
+  };
+  BinWork bw;
 
   // Replayed transforms: the launch sequence of one direction for one
   // (input, output) pair, captured into a HIP graph at the pair's second call
@@ -911,7 +940,7 @@ int check_nodes(const double* k, i64 n) {
 // Node records (NodeRec layout) of the plan's sorted nodes.
 int build_records(nfftm_plan_s& p) {
   const size_t rb = (size_t)node_rec_bytes(p.D, p.dbl() ? sizeof(double) : sizeof(float), p.W);
-  HIPCHK(p.d_rec.alloc(std::max<size_t>(1, (size_t)p.M) * rb));
+  HIPCHK(p.d_rec.ensure(std::max<size_t>(1, (size_t)p.M) * rb));
   HIPCHK(launch_node_records(p.D, p.dbl(), p.W, p.kargs(), p.d_rec.p, p.stream));
   return NFFTM_OK;
 }
@@ -934,25 +963,50 @@ int alloc_grid(nfftm_plan_s& p) {
 int alloc_scratch(nfftm_plan_s& p) {
   const size_t one = std::max<size_t>(1, (size_t)p.nitems) * p.slot_cells() * p.celem();
   p.scap = slice_cap(p, one);
-  HIPCHK(p.d_scratch.alloc((size_t)p.scap * one));
+  HIPCHK(p.d_scratch.ensure((size_t)p.scap * one));
   return NFFTM_OK;
 }
 
 // sort, split each tile's nodes into work items, gather the shifted nodes in
 // tile order.
-int set_nodes(nfftm_plan_s& p, const double* k, i64 M) {
+//
+// k: the caller's host nodes (rows: D rows of M in reversed dimension order,
+// otherwise Julia's D x M), or null to bin the plan's own nodes again.  The
+// range check runs on the device with the first binning kernel; nothing of
+// the plan changes before its result is read.  keep: the work arrays stay
+// with the plan (nodes! is called again and again; a dozen allocations and
+// releases took 0.5 ms of it).
+int set_nodes(nfftm_plan_s& p, const double* k, bool rows, i64 M, bool keep) {
   const int D = p.D;
   if (M < 0 || M > 0x7fffffff) return fail(NFFTM_ERR_UNSUPPORTED, "M = %lld out of range", (long long)M);
-  if (int rc = check_nodes(k, (i64)D * M)) return rc;
-  p.M = M;
-  p.gen++;
-  p.drop_graphs();
-  if (k != p.k.data()) p.k.assign(k, k + (size_t)D * M);
   hipStream_t st = p.stream;
+  nfftm_plan_s::BinWork& w = p.bw;
+  struct Release {
+    nfftm_plan_s& p;
+    bool keep;
+    ~Release() {
+      if (!keep) p.bw.release();
+    }
+  } release{p, keep};
+  if (k) {
+    HIPCHK(w.k.ensure((size_t)D * M));
+    if (M) HIPCHK(hipMemcpyAsync(w.k.p, k, (size_t)D * M * sizeof(double), hipMemcpyHostToDevice, st));
+  } else {
+    rows = p.krows;
+  }
+  const double* kd = k ? w.k.p : p.d_k.p;
+  auto bad_node = [&]() -> int {
+    if (k)
+      if (int rc = check_nodes(k, (i64)D * M)) return rc;
+    return fail(NFFTM_ERR_ARG, "Nodes k need to be within the range [-1/2, 1/2]");
+  };
   BinArgs a;
   std::memset(&a, 0, sizeof a);
   a.D = D;
   a.M = M;
+  a.sd = rows ? -M : 1;
+  a.sj = rows ? 1 : D;
+  const double* k0 = rows ? kd + (i64)(D - 1) * M : kd;
   i64 ntile = 1;
   for (int d = 0; d < 3; ++d) {
     a.Nt[d] = d < D ? (int)p.Nt[d] : 1;
@@ -975,46 +1029,54 @@ int set_nodes(nfftm_plan_s& p, const double* k, i64 M) {
   }
   a.key_bits = 1;
   while (((i64)1 << a.key_bits) < ntile) ++a.key_bits;
-  DevBuf<double> kd;
-  HIPCHK(kd.alloc((size_t)D * M));
-  if (M) HIPCHK(hipMemcpyAsync(kd.p, k, (size_t)D * M * sizeof(double), hipMemcpyHostToDevice, st));
-  HIPCHK(p.d_ks.alloc((size_t)D * M));
-  HIPCHK(p.d_perm.alloc((size_t)M));
   int nitems = 0, nmulti = 0;
+  HIPCHK(w.stats.ensure(4));
+  if (!w.h_stats) HIPCHK(hipHostMalloc((void**)&w.h_stats, 4 * sizeof(int), hipHostMallocDefault));
+  if (!p.tiled) {
+    HIPCHK(launch_check_nodes(kd, (i64)D * M, w.stats.p + 3, st));
+  } else {
+    HIPCHK(w.key_in.ensure((size_t)M));
+    HIPCHK(w.key_out.ensure((size_t)M));
+    HIPCHK(w.idx_in.ensure((size_t)M));
+    HIPCHK(w.cnt.ensure((size_t)ntile + 1));
+    HIPCHK(w.off.ensure((size_t)ntile + 1));
+    HIPCHK(w.ioff.ensure((size_t)ntile + 1));
+    HIPCHK(launch_bin_keys(a, k0, w.key_in.p, w.idx_in.p, w.cnt.p, st));
+    HIPCHK(launch_bin_scan(a, w.cnt.p, w.off.p, w.ioff.p, w.stats.p, st));
+  }
+  HIPCHK(hipMemcpyAsync(w.h_stats, w.stats.p, 4 * sizeof(int), hipMemcpyDeviceToHost, st));
+  HIPCHK(hipStreamSynchronize(st));
+  if (w.h_stats[3]) return bad_node();
+  if (p.tiled) {
+    nitems = w.h_stats[0];
+    nmulti = w.h_stats[1];
+  }
+  // from here on the plan has the new nodes
+  p.M = M;
+  p.gen++;
+  p.drop_graphs();
+  if (k) {
+    p.d_k.swap(w.k);
+    p.krows = rows;
+  }
+  HIPCHK(p.d_perm.ensure((size_t)M));
   if (!p.tiled) {
     HIPCHK(launch_iota(p.d_perm.p, M, st));
-    HIPCHK(launch_bin_ks(a, kd.p, nullptr, p.d_ks.p, st));
-    HIPCHK(p.d_items.alloc(0));
-    HIPCHK(hipStreamSynchronize(st));  // before kd is freed
+  } else if (M) {
+    const size_t tb = bin_sort_temp_bytes(M, a.key_bits);
+    if (!tb) return fail(NFFTM_ERR_HIP, "radix sort of %lld nodes: temporary size query failed", (long long)M);
+    HIPCHK(w.tmp.ensure(tb));
+    HIPCHK(launch_bin_sort(a, w.tmp.p, tb, w.key_in.p, w.key_out.p, w.idx_in.p, p.d_perm.p, st));
+  }
+  HIPCHK(p.d_ks.ensure((size_t)D * M));
+  HIPCHK(launch_bin_ks(a, k0, p.tiled ? p.d_perm.p : nullptr, p.d_ks.p, st));
+  if (p.tiled) {
+    HIPCHK(p.d_items.ensure((size_t)nitems));
+    HIPCHK(p.d_tstart.ensure((size_t)ntile + 1));
+    HIPCHK(p.d_multi.ensure((size_t)nmulti));
+    HIPCHK(launch_bin_items(a, w.off.p, w.ioff.p, p.d_items.p, p.d_tstart.p, p.d_multi.p, w.stats.p + 2, st));
   } else {
-    DevBuf<int> key_in, key_out, idx_in, cnt, off, ioff, stats;
-    HIPCHK(key_in.alloc((size_t)M));
-    HIPCHK(key_out.alloc((size_t)M));
-    HIPCHK(idx_in.alloc((size_t)M));
-    HIPCHK(cnt.alloc((size_t)ntile + 1));
-    HIPCHK(off.alloc((size_t)ntile + 1));
-    HIPCHK(ioff.alloc((size_t)ntile + 1));
-    HIPCHK(stats.alloc(3));
-    HIPCHK(launch_bin_keys(a, kd.p, key_in.p, idx_in.p, cnt.p, st));
-    DevBuf<char> tmp;
-    if (M) {
-      const size_t tb = bin_sort_temp_bytes(M, a.key_bits);
-      if (!tb) return fail(NFFTM_ERR_HIP, "radix sort of %lld nodes: temporary size query failed", (long long)M);
-      HIPCHK(tmp.alloc(tb));
-      HIPCHK(launch_bin_sort(a, tmp.p, tb, key_in.p, key_out.p, idx_in.p, p.d_perm.p, st));
-    }
-    HIPCHK(launch_bin_scan(a, cnt.p, off.p, ioff.p, stats.p, st));
-    int hs[2] = {0, 0};
-    HIPCHK(hipMemcpyAsync(hs, stats.p, sizeof hs, hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
-    nitems = hs[0];
-    nmulti = hs[1];
-    HIPCHK(p.d_items.alloc((size_t)nitems));
-    HIPCHK(p.d_tstart.alloc((size_t)ntile + 1));
-    HIPCHK(p.d_multi.alloc((size_t)nmulti));
-    HIPCHK(launch_bin_items(a, off.p, ioff.p, p.d_items.p, p.d_tstart.p, p.d_multi.p, stats.p + 2, st));
-    HIPCHK(launch_bin_ks(a, kd.p, p.d_perm.p, p.d_ks.p, st));
-    HIPCHK(hipStreamSynchronize(st));  // before the temporaries are freed
+    HIPCHK(p.d_items.alloc(0));
   }
   p.nitems = nitems;
   p.nmulti = nmulti;
@@ -1037,14 +1099,30 @@ int set_nodes(nfftm_plan_s& p, const double* k, i64 M) {
     // plan builds its records then)
     if (p.sorted_io()) p.d_rec.reset();
     else if (int rc = build_records(p)) return rc;
-    p.d_iperm.reset();
-    p.d_fsort.reset();
     if (p.sorted_io() && M > 0) {
-      HIPCHK(p.d_fsort.alloc((size_t)p.scap * M * p.celem()));
-      HIPCHK(p.d_iperm.alloc((size_t)M));
+      HIPCHK(p.d_fsort.ensure((size_t)p.scap * M * p.celem()));
+      HIPCHK(p.d_iperm.ensure((size_t)M));
       HIPCHK(launch_inv_perm(p.d_perm.p, p.d_iperm.p, M, p.stream));
     }
   }
+  return NFFTM_OK;
+}
+
+// The plan's nodes as Julia's D x M matrix.
+int host_nodes(const nfftm_plan_s& p, std::vector<double>* k) {
+  const size_t n = (size_t)p.D * p.M;
+  std::vector<double> h(n);
+  if (n) {
+    HIPCHK(hipStreamSynchronize(p.stream));
+    HIPCHK(hipMemcpy(h.data(), p.d_k.p, n * sizeof(double), hipMemcpyDeviceToHost));
+  }
+  if (!p.krows) {
+    *k = std::move(h);
+    return NFFTM_OK;
+  }
+  k->resize(n);
+  for (i64 j = 0; j < p.M; ++j)
+    for (int d = 0; d < p.D; ++d) (*k)[(size_t)(d + p.D * j)] = h[(size_t)(j + (p.D - 1 - d) * p.M)];
   return NFFTM_OK;
 }
 
@@ -1385,7 +1463,7 @@ int create_impl(nfftm_plan_s& p, const double* k) {
   p.f1 = !p.pfft && !p.mix && p.D == 1 && !(p.flags & NFFTM_FLAG_ROCFFT) &&
          fft1_factor(p.Nt[0], p.N[0], p.dbl(), &p.f1n1, &p.f1Lm);
   if (int rc = build_tables(p)) return rc;
-  if (int rc = set_nodes(p, k, p.M)) return rc;
+  if (int rc = set_nodes(p, k, false, p.M, false)) return rc;
   if (int rc = alloc_grid(p)) return rc;
   p.fft.reset(new FFTStage());
   if (int rc = p.fft->build(p.D, p.Nt, p.dbl())) return rc;
@@ -1503,7 +1581,8 @@ int time_gridding(nfftm_plan_s& p, void* fh, double* ms) {
 int tune_plan(nfftm_plan_s& p, int maxNT, std::vector<TuneChoice>* log) {
   if (!p.tiled || p.M == 0) return NFFTM_OK;
   const i64 Mfull = p.M;
-  const std::vector<double> kfull = p.k;
+  std::vector<double> kfull;
+  if (int rc = host_nodes(p, &kfull)) return rc;
   const i64 stride = (Mfull + (1 << 20) - 1) >> 20;
   std::vector<double> ksub;
   if (stride > 1) {
@@ -1539,7 +1618,7 @@ int tune_plan(nfftm_plan_s& p, int maxNT, std::vector<TuneChoice>* log) {
       p.NT = best.NT;
     }
     const std::string err = g_err;
-    const int rc2 = set_nodes(p, kfull.data(), Mfull);
+    const int rc2 = set_nodes(p, kfull.data(), false, Mfull, false);
     if (rc != NFFTM_OK) {
       g_err = err;  // report the tuning failure, not the restore
       return rc;
@@ -1550,7 +1629,7 @@ int tune_plan(nfftm_plan_s& p, int maxNT, std::vector<TuneChoice>* log) {
     const bool ok = p.D == 3 ? set_tile3(p, c.first) : set_tile_shape(p, c.first);
     if (!ok || !tiles_ok(p)) continue;
     if (c.first != binned) {
-      if (int rc = set_nodes(p, ktune, Mtune)) return restore(rc);
+      if (int rc = set_nodes(p, ktune, false, Mtune, true)) return restore(rc);
       binned = c.first;
     }
     p.NT = c.second;
@@ -1955,9 +2034,16 @@ int nfftm_nodes(nfftm_plan p, const double* k_host, int64_t M) {
   g_err.clear();
   if (!p) return fail(NFFTM_ERR_ARG, "plan is NULL");
   if (M > 0 && !k_host) return fail(NFFTM_ERR_ARG, "k is NULL");
-  if (int rc = check_nodes(k_host, (i64)p->D * M)) return rc;
   HIPCHK(hipStreamSynchronize(p->stream));
-  return set_nodes(*p, k_host, M);
+  return set_nodes(*p, k_host, false, M, true);
+}
+
+int nfftm_nodes_rows(nfftm_plan p, const double* k_host, int64_t M) {
+  g_err.clear();
+  if (!p) return fail(NFFTM_ERR_ARG, "plan is NULL");
+  if (M > 0 && !k_host) return fail(NFFTM_ERR_ARG, "k is NULL");
+  HIPCHK(hipStreamSynchronize(p->stream));
+  return set_nodes(*p, k_host, true, M, true);
 }
 
 }  // extern "C"
@@ -2312,7 +2398,9 @@ int nfftm_plan_copy(nfftm_plan src, nfftm_plan* dst) {
   p->Bsl = src->Bsl;
   p->Asl = src->Asl;
   for (int d = 0; d < MAXD; ++d) p->Nfull[d] = src->Nfull[d];
-  if (int rc = create_impl(*p, src->k.data())) return rc;
+  std::vector<double> k;
+  if (int rc = host_nodes(*src, &k)) return rc;
+  if (int rc = create_impl(*p, k.data())) return rc;
   std::memcpy(p->timing, src->timing, sizeof p->timing);
   *dst = p.release();
   return NFFTM_OK;
@@ -2352,11 +2440,11 @@ int nfftm_plan_set_tiles(nfftm_plan p, int tile, int threads) {
   const bool ok = p->D == 3 ? (tile == 0 || tile == 1) && set_tile3(*p, tile) : tile > 0 && set_tile_shape(*p, tile);
   if (!ok || !tiles_ok(*p)) {
     choose_tiles(*p);
-    if (int rc = set_nodes(*p, p->k.data(), p->M)) return rc;
+    if (int rc = set_nodes(*p, nullptr, false, p->M, false)) return rc;
     return fail(NFFTM_ERR_UNSUPPORTED, "tile %d does not fit this plan", tile);
   }
   p->NT = threads;
-  return set_nodes(*p, p->k.data(), p->M);
+  return set_nodes(*p, nullptr, false, p->M, false);
 }
 
 int nfftm_tile_shape(nfftm_plan p, int* tile, int* threads) {

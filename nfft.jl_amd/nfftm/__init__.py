@@ -359,11 +359,11 @@ class NFFTPlan:
         if self.params["sortNodes"]:
             order = np.lexsort(k)
             k[:] = k[:, order]
-        kj = np.ascontiguousarray(k[::-1].T, dtype=np.float64)
+        kr = np.ascontiguousarray(k, dtype=np.float64)
         torch.cuda.current_stream().synchronize()
-        _check(self._lib.nfftm_nodes(self._handle,
-                                     kj.ctypes.data_as(ctypes.POINTER(ctypes.c_double)),
-                                     k.shape[1]))
+        _check(self._lib.nfftm_nodes_rows(self._handle,
+                                          kr.ctypes.data_as(ctypes.POINTER(ctypes.c_double)),
+                                          k.shape[1]))
         self.k = k
         self._read_sizes()
         return self

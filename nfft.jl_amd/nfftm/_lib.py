@@ -21,7 +21,7 @@ R32, R64, C32, C64, R16, C16 = range(6)  # element types of the typed stage oper
 
 # every symbol include/nfftm.h declares
 EXPORTS = (
-    "nfftm_plan_create", "nfftm_plan_create_dims", "nfftm_nodes", "nfftm_forward", "nfftm_adjoint",
+    "nfftm_plan_create", "nfftm_plan_create_dims", "nfftm_nodes", "nfftm_nodes_rows", "nfftm_forward", "nfftm_adjoint",
     "nfftm_deconvolve", "nfftm_deconvolve_transpose", "nfftm_convolve",
     "nfftm_convolve_transpose", "nfftm_convolve_typed", "nfftm_convolve_transpose_typed", "nfftm_fft", "nfftm_sizes", "nfftm_grid",
     "nfftm_timing", "nfftm_set_timing", "nfftm_profile", "nfftm_profile_read",
@@ -55,6 +55,7 @@ def load():
     L.nfftm_plan_create.argtypes = [ctypes.POINTER(vp), i, i, pi64, i64, pd, i, d, i, i, i, vp]
     L.nfftm_plan_create_dims.argtypes = [ctypes.POINTER(vp), i, i, pi64, i, i, i64, pd, i, d, i, i, i, vp]
     L.nfftm_nodes.argtypes = [vp, pd, i64]
+    L.nfftm_nodes_rows.argtypes = [vp, pd, i64]
     L.nfftm_grad_nodes.argtypes = [vp, vp, vp, vp]
     L.nfftm_grad_nodes_grid.argtypes = [vp, vp, vp, vp]
     L.nfftm_plan_tune.argtypes = [vp]
