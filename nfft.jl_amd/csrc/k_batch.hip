@@ -44,9 +44,10 @@ __global__ __launch_bounds__(NT) void k_spread_batch(const KArgs* __restrict__ k
   }
 }
 
-// Fold of a batch: work entry {slot, first, end, 0} -- grid rows for D = 2,
-// points of the single row for D = 1; the workgroup sums the covering
-// scratch slots of every point.
+// Fold of a batch: work entry {slot, first, end, 0} -- points of the single
+// row for D = 1; D = 2: points of the tile `end` from `first` on (a.blocked3),
+// else grid rows.  The workgroup sums the covering scratch slots of every
+// point.
 template <typename R, int D>
 __global__ __launch_bounds__(256) void k_fold_batch(const KArgs* __restrict__ ka, const int4* __restrict__ work,
                                                     int nwork, void* const* __restrict__ grids) {
@@ -59,6 +60,10 @@ __global__ __launch_bounds__(256) void k_fold_batch(const KArgs* __restrict__ ka
     const int ny = D >= 2 ? a.Nt[1] : 1;
     int t1[3] = {0, 0, 0}, p1[3] = {0, 0, 0}, t2[3] = {0, 0, 0}, p2[3] = {0, 0, 0};
     int n1 = 1, n2 = 1;
+    if (D == 2 && a.blocked3) {
+      fold2_point<R>(a, scr, grid, e.z, e.y + (int)threadIdx.x);
+      continue;
+    }
     if (D == 1) {
       for (int x = e.y + threadIdx.x; x < e.z; x += 256)
         grid[x] = fold_sum<R, D>(a, scr, x, n1, t1, p1, n2, t2, p2);

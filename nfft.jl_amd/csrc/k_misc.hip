@@ -538,15 +538,18 @@ hipError_t launch_gather_nodes(bool dbl, const void* in, long long is, const int
   return hipGetLastError();
 }
 
-size_t tile_lds_bytes(int D, bool dbl, int W, int tileElems) {
-  int NB;
-  if (dbl) NB = D == 1 ? Batch<1, double>::NB : D == 2 ? Batch<2, double>::NB : Batch<3, double>::NB;
-  else NB = D == 1 ? Batch<1, float>::NB : D == 2 ? Batch<2, float>::NB : Batch<3, float>::NB;
-  return tile_layout_bytes(D, dbl ? sizeof(double) : sizeof(float), W, tileElems, NB);
+size_t tile_lds_bytes(bool dbl, int tileElems) {
+  return tile_layout_bytes(dbl ? sizeof(double) : sizeof(float), tileElems);
 }
 
 hipError_t launch_fold(int D, bool dbl, int W, const KArgs& a, hipStream_t s, void* grid) {
   if (D == 3) return launch_fold_d3(dbl, W, a, s, grid);
+  if (D == 2 && a.blocked3) {
+    const dim3 g((unsigned)a.ntile_all, (unsigned)((a.T[0] * a.T[1] + 255) / 256), (unsigned)a.nsl);
+    if (dbl) hipLaunchKernelGGL(k_fold2<double>, g, dim3(256), 0, s, a, (double2*)grid);
+    else hipLaunchKernelGGL(k_fold2<float>, g, dim3(256), 0, s, a, (float2*)grid);
+    return hipGetLastError();
+  }
   long long rows = 1;
   for (int d = 1; d < D; ++d) rows *= a.Nt[d];
   const dim3 g((a.Nt[0] + 255) / 256, (unsigned)std::min<long long>(rows, 65535), a.nsl), blk(256);

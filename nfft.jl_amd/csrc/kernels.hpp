@@ -90,7 +90,7 @@ struct KArgs {
   int Sx, Sxy;     // LDS strides of the padded tile (elements)
   int tileElems;   // elements of one LDS plane
   int padCells;    // Pd[0]*Pd[1]*Pd[2]
-  FastDiv divP0, divP1, divNtx;
+  FastDiv divP0, divT0;
   // window
   const void* lut;  // R[LUTSize + 2]
   long long scale;  // LUTSize / m, a power of two
@@ -110,7 +110,8 @@ struct KArgs {
   int nitems;
   const char* rec;    // node records in sorted order (NodeRec layout), tiled plans
   int recBytes;
-  int blocked3;       // 3-D scratch slots stored as 27 halo/interior blocks
+  int blocked3;       // 3-D scratch slots stored as 27 halo/interior blocks; 2-D: every grid
+                      // point is covered by its own tile and neighbouring ones only (k_fold2)
   int tvar;           // 3-D tile geometry variant (compile-time tile edge)
   int fix2;           // FP32 2-D spreading accumulates packed fixed point (one
                       // 64-bit LDS atomic per tap) instead of two FP64 planes
@@ -349,36 +350,19 @@ __host__ inline int node_rec_bytes(int D, size_t sizeofR, int W) {
   return (int)((D * W * sizeofR + 8 + 15) & ~(size_t)15);
 }
 
-// LDS layout of the D <= 2 tile kernels: tile, node records of one batch,
-// node values of one batch (spreading).
-template <typename R, int D, int W>
-struct TileLayout {
-  // the spreading tile of D <= 2 accumulates in FP64 in both precisions
-  static constexpr size_t ACC = D <= 2 ? sizeof(double) : sizeof(R);
-  static __host__ __device__ size_t rec_off(int tileElems) { return (2 * (size_t)tileElems * ACC + 15) & ~(size_t)15; }
-  static __host__ __device__ size_t fv_off(int tileElems, int NB) {
-    return rec_off(tileElems) + (size_t)NB * NodeRec<R, D, W>::BYTES;
-  }
-  static __host__ __device__ size_t bytes(int tileElems, int NB) {
-    return fv_off(tileElems, NB) + (size_t)NB * 2 * sizeof(R);
-  }
-};
-
-// The same layout size for a runtime stencil width (host side).
-__host__ inline size_t tile_layout_bytes(int D, size_t sizeofR, int W, int tileElems, int NB) {
-  const size_t acc = D <= 2 ? sizeof(double) : sizeofR;
-  const size_t o = (2 * (size_t)tileElems * acc + 15) & ~(size_t)15;
-  return o + (size_t)NB * node_rec_bytes(D, sizeofR, W) + (size_t)NB * 2 * sizeofR;
+// LDS layout of the D <= 2 tile kernels: the tile (spreading: FP64 planes or
+// packed fixed point, in both precisions at most two doubles per cell), then
+// the node values of one batch (spreading).
+constexpr int NBV = 512;  // node values of a batch at most
+__host__ __device__ __forceinline__ size_t tile_fv_off(int tileElems) {
+  return (2 * (size_t)tileElems * sizeof(double) + 15) & ~(size_t)15;
+}
+__host__ inline size_t tile_layout_bytes(size_t sizeofR, int tileElems) {
+  return tile_fv_off(tileElems) + NBV * 2 * sizeofR;
 }
 
 // Nodes of one 3-D work item at most (items are chunks of one tile's nodes).
 constexpr int ITEM3 = 1024;
-
-// Nodes per phase-A batch.
-template <int D, typename R>
-struct Batch {
-  static constexpr int NB = D == 3 ? (sizeof(R) == 4 ? 256 : 128) : 256;
-};
 
 __device__ __forceinline__ void tile_origin(const KArgs& a, int D, int tile, int* t0) {
   int r = tile;
@@ -427,24 +411,31 @@ __global__ __launch_bounds__(256) void k_node_records(KArgs a, char* __restrict_
   for (int i = 0; i < N::BYTES / 16; ++i) out[i] = make_uint4(u[4 * i], u[4 * i + 1], u[4 * i + 2], u[4 * i + 3]);
 }
 
-// Phase A: copy the records of nodes [b0, b0 + nb) into LDS (16-byte
-// blocks); for spreading also gather their values fhat[pj] * scale.
-template <typename R, int D, int W, int NT, bool SPREAD>
-__device__ __forceinline__ void phase_a(const KArgs& a, const typename cpx<R>::T* __restrict__ fhat, int b0, int nb,
-                                        char* lrec, typename cpx<R>::T* fv, R scale) {
-  using N = NodeRec<R, D, W>;
-  const uint4* src = (const uint4*)(a.rec + (size_t)b0 * N::BYTES);
-  uint4* dst = (uint4*)lrec;
-  const int n16 = nb * (N::BYTES / 16);
-  for (int i = threadIdx.x; i < n16; i += NT) dst[i] = src[i];
-  if (SPREAD) {
-    for (int n = threadIdx.x; n < nb; n += NT) {
-      const int jj = ((const int*)(a.rec + (size_t)(b0 + n) * N::BYTES + N::WBYTES))[1];
-      const typename cpx<R>::T v = fhat[(long long)jj * a.fst];
-      fv[n] = typename cpx<R>::T{v.x * scale, v.y * scale};
+// The record of one node as a lane of its group holds it (D <= 2): the
+// dimension-1 weight of the lane's column, the dimension-2 weights, the packed
+// cell and the caller's index.  Read straight from global memory, one step
+// ahead of its use: the lanes of a group read the same words, a wavefront's
+// groups consecutive records.  (Copying the records through LDS took a block
+// copy, a barrier and, per node, as many LDS reads as the taps have adds; two
+// or four steps ahead: more registers, the same or a longer time.)
+template <typename R, int D, int W>
+struct NodeTaps {
+  R w1, w2[D == 2 ? W : 1];
+  unsigned pk;
+  int pj;
+  __device__ __forceinline__ void load(const char* __restrict__ rec, long long j, int lx) {
+    using N = NodeRec<R, D, W>;
+    const char* r = rec + (size_t)j * N::BYTES;
+    w1 = ((const R*)r)[lx];
+    if constexpr (D == 2) {
+#pragma unroll
+      for (int l = 0; l < W; ++l) w2[l] = ((const R*)r)[W + l];
     }
+    const int2 q = *(const int2*)(r + N::WBYTES);
+    pk = (unsigned)q.x;
+    pj = q.y;
   }
-}
+};
 
 // Fields of a record in LDS.
 template <typename R, int D, int W>
@@ -500,42 +491,67 @@ struct SpreadCell<double> {  // two FP64 planes
 
 // One work item (<= CH nodes of one tile, D <= 2) of spreading: the padded
 // tile is accumulated in LDS -- FP64 adds of the data-precision products, one
-// rounding per term -- and written to the item's slot of `scratch`.
+// rounding per term, or packed fixed point -- and written to the item's slot
+// of `scratch`.  W lanes per node (one per dimension-1 column, 64 / W nodes
+// per wavefront step), each walking dimension 2.
+//
+// A plan of ordinary size has about one item per resident workgroup, so the
+// time of an item is the chain of its memory latencies: item, then (caller
+// index, node value) beside (first records), one barrier, taps, flush.  2 10^5
+// radial nodes on 512^2 points, FP32, m = 4: 16.2 -> 13.2 us; 32 slices of
+// 1.2 10^5 nodes: 171 -> 150 us.  FP64 is bound by its two LDS adds per tap.
 template <typename R, int D, int W, int NT>
 __device__ __forceinline__ void spread_tile_item(const KArgs& a, int item,
                                                  const typename cpx<R>::T* __restrict__ fhat,
                                                  typename cpx<R>::T* __restrict__ scratch) {
   static_assert(D <= 2, "3-D spreading lives in k_tile3.hip");
   using C = typename cpx<R>::T;
-  using L = TileLayout<R, D, W>;
   using A = double;
-  constexpr int NB = Batch<D, R>::NB;
-  constexpr int NW = NT / 64;
+  constexpr int NW = NT / 64, NB = NT < NBV ? NT : NBV;
+  // FP32 2-D: the values of all nodes of an item (at most 2048) in registers,
+  // for the fixed-point bound; otherwise one batch ahead
+  constexpr bool HOLD = sizeof(R) == 4 && D == 2;
+  constexpr int HPT = HOLD ? 2048 / NB : 1;
   constexpr unsigned LM = NodeRec<R, D, W>::LOCBITS >= 32 ? 0xFFFFFFFFu : (1u << NodeRec<R, D, W>::LOCBITS) - 1u;
+  constexpr int NPW = 64 / W;
   extern __shared__ __align__(16) char smem[];
   const int4 it = a.items[item];
   char* tile = smem;
-  char* lrec = smem + L::rec_off(a.tileElems);
-  C* fv = (C*)(smem + L::fv_off(a.tileElems, NB));
+  C* fv = (C*)(smem + tile_fv_off(a.tileElems));
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int slot = lane / W, lx = lane - slot * W;
+  const bool lane_on = slot < NPW;
+  const int tid = threadIdx.x;
 
-  for (int i = threadIdx.x; i < 2 * a.tileElems; i += NT) ((A*)tile)[i] = 0;
+  R hre[HPT], him[HPT];
+#pragma unroll
+  for (int h = 0; h < HPT; ++h) {
+    const int j = it.y + tid + h * NB;
+    C v{0, 0};
+    if (tid < NB && j < it.z) v = fhat[(long long)a.perm[j] * a.fst];
+    hre[h] = v.x;
+    him[h] = v.y;
+  }
+  int n = it.y + wave * NPW + slot;  // the lane's node
+  NodeTaps<R, D, W> nx;
+  nx.load(a.rec, lane_on && n < it.z ? n : it.y, lane_on ? lx : 0);
 
   // FP32 2-D with fix2: packed 32+32-bit fixed point in the first tileElems
   // 64-bit words, scale s = 2^(30 - e) from a strict bound of the item's
   // sums, B = sum_j |f_j|_inf * wmaxD < 2^e (as the 3-D FP32 kernel); one
   // ds_add_u64 per tap instead of two ds_add_f64
-  const bool fix = sizeof(R) == 4 && D == 2 && a.fix2;
+  const bool fix = HOLD && a.fix2;
+  {
+    const int nz = fix ? a.tileElems : 2 * a.tileElems;
+    for (int i = tid; i < nz; i += NT) ((A*)tile)[i] = 0;
+  }
   R fscale = 1, inv = 1;
   if (fix) {
     R part = 0;
-    for (int j = it.y + (int)threadIdx.x; j < it.z; j += NT) {
-      const int jj = ((const int*)(a.rec + (size_t)j * NodeRec<R, D, W>::BYTES + NodeRec<R, D, W>::WBYTES))[1];
-      const C v = fhat[(long long)jj * a.fst];
-      part += fmax(fabs(v.x), fabs(v.y));
-    }
+#pragma unroll
+    for (int h = 0; h < HPT; ++h) part += fmax(fabs(hre[h]), fabs(him[h]));
     part = group_sum<64>(part);
-    R* red = (R*)lrec;
+    R* red = (R*)fv;
     if (lane == 0) red[wave] = part;
     __syncthreads();
     double B = 0;
@@ -552,46 +568,56 @@ __device__ __forceinline__ void spread_tile_item(const KArgs& a, int item,
       fscale = 0;
       inv = (R)NAN;
     }
+    __syncthreads();  // before fv takes the values
   }
+  const R sc = (R)a.oscale * fscale;
 
-  constexpr int G = LanesPerNode<W>::value;
-  constexpr int NPW = 64 / G;
-  const int slot = lane / G, lx = lane & (G - 1);
-  for (int b0 = it.y; b0 < it.z; b0 += NB) {
-    const int nb = min(NB, it.z - b0);
+#pragma unroll(HOLD ? HPT : 1)
+  for (int h = 0; h < (HOLD ? HPT : 1 << 20); ++h) {
+    const int b0 = it.y + h * NB;
+    if (b0 >= it.z) break;
+    const int b1 = min(b0 + NB, it.z);
+    if (tid < NB) fv[tid] = C{hre[HOLD ? h : 0] * sc, him[HOLD ? h : 0] * sc};
     __syncthreads();
-    phase_a<R, D, W, NT, true>(a, fhat, b0, nb, lrec, fv, (R)a.oscale * fscale);
-    __syncthreads();
-    for (int n0 = wave * NPW; n0 < nb; n0 += NW * NPW) {
-      const int n = n0 + slot;
-      if (n < nb && lx < W) {
-        const C f = fv[n];
-        const R* w = rec_w<R, D, W>(lrec, n);
-        const unsigned pk = rec_loc<R, D, W>(lrec, n);
-        const R w1 = w[lx];
-        const R vr = f.x * w1, vi = f.y * w1;
+    if constexpr (!HOLD) {  // the next batch's values
+      const int j = b0 + NB + tid;
+      C v{0, 0};
+      if (tid < NB && j < it.z) v = fhat[(long long)a.perm[j] * a.fst];
+      hre[0] = v.x;
+      him[0] = v.y;
+    }
+    for (int n0 = b0 + wave * NPW; n0 < b1; n0 += NW * NPW) {
+      n = n0 + slot;
+      const bool on = lane_on && n < b1;
+      const NodeTaps<R, D, W> c = nx;
+      // the next step's node: in this batch, or the wavefront's first of the
+      // next one
+      const int m0 = n0 + NW * NPW < b1 ? n0 + NW * NPW : b0 + NB + wave * NPW;
+      const int m = m0 + slot;
+      nx.load(a.rec, lane_on && m < it.z ? m : it.y, lane_on ? lx : 0);
+      if (on) {
+        const C f = fv[n - b0];
+        const R vr = f.x * c.w1, vi = f.y * c.w1;
         if constexpr (D == 2) {
-          const int base = ((int)(pk & LM) + lx) + a.Sx * (int)(pk >> 16);
+          const int base = ((int)(c.pk & LM) + lx) + a.Sx * (int)(c.pk >> 16);
           if (fix) {
 #pragma unroll
-            for (int ly = 0; ly < W; ++ly) {
-              const R w2 = w[W + ly];
-              SpreadCell<float>::add(tile, a.tileElems, base + a.Sx * ly, (float)(vr * w2), (float)(vi * w2));
-            }
+            for (int ly = 0; ly < W; ++ly)
+              SpreadCell<float>::add(tile, a.tileElems, base + a.Sx * ly, (float)(vr * c.w2[ly]),
+                                     (float)(vi * c.w2[ly]));
           } else {
 #pragma unroll
-            for (int ly = 0; ly < W; ++ly) {
-              const R w2 = w[W + ly];
-              SpreadCell<A>::add(tile, a.tileElems, base + a.Sx * ly, (A)(vr * w2), (A)(vi * w2));
-            }
+            for (int ly = 0; ly < W; ++ly)
+              SpreadCell<A>::add(tile, a.tileElems, base + a.Sx * ly, (A)(vr * c.w2[ly]), (A)(vi * c.w2[ly]));
           }
         } else {
-          SpreadCell<A>::add(tile, a.tileElems, (int)pk + lx, (A)vr, (A)vi);
+          SpreadCell<A>::add(tile, a.tileElems, (int)c.pk + lx, (A)vr, (A)vi);
         }
       }
     }
+    __syncthreads();
   }
-  __syncthreads();
+  if (it.y >= it.z) __syncthreads();
 
   // padded tile -> this item's scratch slot (dense, px fastest), plain stores
   C* out = scratch + (size_t)item * a.padCells;
@@ -704,77 +730,163 @@ __global__ __launch_bounds__(256) void k_fold(KArgs a, typename cpx<R>::T* __res
   }
 }
 
+// 2-D fold where every tile has at least m cells per dimension: a point is
+// covered by its own tile and the eight around it only.  One workgroup per
+// tile, a thread per point: the item ranges of the nine tiles are uniform and
+// read together, then the (at most four) covering values together, where
+// fold_sum walks the covering pairs one dependent load after the other
+// (512^2 points, FP32, radial nodes: 12.9 -> 9 us).
+template <typename R>
+__device__ __forceinline__ void fold2_point(const KArgs& a, const typename cpx<R>::T* __restrict__ scr,
+                                            typename cpx<R>::T* __restrict__ grid, int tile, int c) {
+  using C = typename cpx<R>::T;
+  const int ntx = a.ntiles[0], nty = a.ntiles[1], oy = tile / ntx, ox = tile - oy * ntx;
+  const int ly = (int)fdiv((uint32_t)c, a.divT0), lx = c - ly * a.T[0];
+  const int x = ox * a.T[0] + lx, y = oy * a.T[1] + ly;
+  const bool in = ly < a.T[1] && x < a.Nt[0] && y < a.Nt[1];
+  int i0[9], i1[9], off[9];
+#pragma unroll
+  for (int q = 0; q < 9; ++q) {
+    const int dx = q % 3 - 1, dy = q / 3 - 1;
+    int ux = ox + dx, uy = oy + dy, ix = x, iy = y;
+    if (ux < 0) ux += ntx, ix += a.Nt[0];
+    if (ux >= ntx) ux -= ntx, ix -= a.Nt[0];
+    if (uy < 0) uy += nty, iy += a.Nt[1];
+    if (uy >= nty) uy -= nty, iy -= a.Nt[1];
+    const int t = ux + ntx * uy;
+    i0[q] = a.tstart[t];
+    i1[q] = a.tstart[t + 1];
+    const int px = ix - ux * a.T[0] + a.m - 1, py = iy - uy * a.T[1] + a.m - 1;
+    off[q] = in && px >= 0 && px < a.Pd[0] && py >= 0 && py < a.Pd[1] ? px + a.Pd[0] * py : -1;
+  }
+  C v[9];
+#pragma unroll
+  for (int q = 0; q < 9; ++q) {
+    v[q] = C{0, 0};
+    if (i1[q] > i0[q] && off[q] >= 0) v[q] = scr[(size_t)i0[q] * a.padCells + off[q]];
+  }
+  R sr = 0, si = 0;
+#pragma unroll
+  for (int q = 0; q < 9; ++q) {
+    sr += v[q].x;
+    si += v[q].y;
+    for (int itm = i0[q] + 1; itm < i1[q]; itm += 8) {  // crowded tiles, eight items in flight
+      C w[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        w[u] = C{0, 0};
+        if (itm + u < i1[q] && off[q] >= 0) w[u] = scr[(size_t)(itm + u) * a.padCells + off[q]];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        sr += w[u].x;
+        si += w[u].y;
+      }
+    }
+  }
+  if (in) grid[(long long)y * a.Nt[0] + x] = C{sr, si};
+}
+
+template <typename R>
+__global__ __launch_bounds__(256) void k_fold2(KArgs a, typename cpx<R>::T* __restrict__ grid) {
+  using C = typename cpx<R>::T;
+  fold2_point<R>(a, (const C*)a.scratch + slice_scratch(a, blockIdx.z), grid + slice_slot(a, blockIdx.z),
+                 (int)blockIdx.x, (int)(blockIdx.y * 256 + threadIdx.x));
+}
+
 // ---------------------------------------------------------------------------
 // Interpolation
 // ---------------------------------------------------------------------------
 // One work item of interpolation (D <= 2): stage the padded tile, gather
-// every node with G lanes per node.
+// every node with G lanes per node (one per dimension-1 column); the first
+// records are read while the tile is staged, each later one a step ahead
+// (32 slices of 1.2 10^5 nodes, FP32, m = 4: 130 -> 121 us).
 template <typename R, int D, int W, int NT>
 __device__ __forceinline__ void interp_tile_item(const KArgs& a, int item,
                                                  const typename cpx<R>::T* __restrict__ grid,
                                                  typename cpx<R>::T* __restrict__ fhat) {
   static_assert(D <= 2, "3-D interpolation lives in k_tile3.hip");
   using C = typename cpx<R>::T;
-  using L = TileLayout<R, D, W>;
-  constexpr int NB = Batch<D, R>::NB;
   constexpr int NW = NT / 64;
   constexpr unsigned LM = NodeRec<R, D, W>::LOCBITS >= 32 ? 0xFFFFFFFFu : (1u << NodeRec<R, D, W>::LOCBITS) - 1u;
+  constexpr int G = LanesPerNode<W>::value;
+  constexpr int NPW = 64 / G;
   extern __shared__ __align__(16) char smem[];
   const int4 it = a.items[item];
   C* tile = (C*)smem;
-  char* lrec = smem + L::rec_off(a.tileElems);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int slot = lane / G, lx = lane & (G - 1), lw = min(lx, W - 1);
+  NodeTaps<R, D, W> nx;
+  {
+    const int n = it.y + wave * NPW + slot;
+    nx.load(a.rec, n < it.z ? n : it.y, lw);
+  }
   int t0[3] = {0, 0, 0};
   tile_origin(a, D, it.x, t0);
 
-  // stage the padded tile
-  for (int i = threadIdx.x; i < a.padCells; i += NT) {
-    int px = i, py = 0;
-    if (D >= 2) {
-      const int q = (int)fdiv((uint32_t)i, a.divP0);
-      px = i - q * a.Pd[0];
-      py = q;
-    }
-    long long gi = wrapidx((long long)t0[0] - a.m + 1 + px, a.Nt[0]);
-    if (D >= 2) gi += wrapidx((long long)t0[1] - a.m + 1 + py, a.Nt[1]) * a.gstr[1];
-    tile[px + a.Sx * py] = grid[gi];
-  }
-
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  constexpr int G = LanesPerNode<W>::value;
-  constexpr int NPW = 64 / G;
-  const int slot = lane / G, lx = lane & (G - 1);
-  for (int b0 = it.y; b0 < it.z; b0 += NB) {
-    const int nb = min(NB, it.z - b0);
-    __syncthreads();
-    phase_a<R, D, W, NT, false>(a, nullptr, b0, nb, lrec, nullptr, (R)1);
-    __syncthreads();
-    for (int n0 = wave * NPW; n0 < nb; n0 += NW * NPW) {
-      const int n = n0 + slot;
-      R ar = 0, ai = 0;
-      if (n < nb && lx < W) {
-        const R* w = rec_w<R, D, W>(lrec, n);
-        const unsigned pk = rec_loc<R, D, W>(lrec, n);
-        if constexpr (D == 2) {
-          const int base = ((int)(pk & LM) + lx) + a.Sx * (int)(pk >> 16);
+  // stage the padded tile (within one period: at most one wrap per index),
+  // ST cells per thread in flight
+  constexpr int ST = 2;
+  for (int i0 = threadIdx.x; i0 < a.padCells; i0 += ST * NT) {
+    C v[ST];
+    int li[ST];
 #pragma unroll
-          for (int ly = 0; ly < W; ++ly) {
-            const C v = tile[base + a.Sx * ly];
-            ar = fma(w[W + ly], v.x, ar);
-            ai = fma(w[W + ly], v.y, ai);
-          }
-          ar *= w[lx];
-          ai *= w[lx];
-        } else {
-          const C v = tile[(int)pk + lx];
-          ar = w[lx] * v.x;
-          ai = w[lx] * v.y;
-        }
+    for (int u = 0; u < ST; ++u) {
+      const int i = i0 + u * NT;
+      const bool ok = i < a.padCells;
+      int px = ok ? i : 0, py = 0;
+      if (D >= 2) {
+        const int q = (int)fdiv((uint32_t)px, a.divP0);
+        px -= q * a.Pd[0];
+        py = q;
       }
-      ar = group_sum<G>(ar);
-      ai = group_sum<G>(ai);
-      if (lx == 0 && n < nb)
-        fhat[(long long)rec_pj<R, D, W>(lrec, n) * a.fst] = C{ar * (R)a.oscale, ai * (R)a.oscale};
+      int gx = t0[0] - a.m + 1 + px;
+      gx += gx < 0 ? a.Nt[0] : 0;
+      gx -= gx >= a.Nt[0] ? a.Nt[0] : 0;
+      long long gi = gx;
+      if (D >= 2) {
+        int gy = t0[1] - a.m + 1 + py;
+        gy += gy < 0 ? a.Nt[1] : 0;
+        gy -= gy >= a.Nt[1] ? a.Nt[1] : 0;
+        gi += (long long)gy * a.Nt[0];
+      }
+      v[u] = grid[gi];
+      li[u] = ok ? px + a.Sx * py : -1;
     }
+#pragma unroll
+    for (int u = 0; u < ST; ++u)
+      if (li[u] >= 0) tile[li[u]] = v[u];
+  }
+  __syncthreads();
+
+  const R osc = (R)a.oscale;
+  for (int n0 = it.y + wave * NPW; n0 < it.z; n0 += NW * NPW) {
+    const int n = n0 + slot;
+    const bool on = n < it.z;
+    const NodeTaps<R, D, W> c = nx;
+    const int m = n + NW * NPW;
+    nx.load(a.rec, m < it.z ? m : it.y, lw);
+    R ar = 0, ai = 0;
+    if (on && lx < W) {
+      if constexpr (D == 2) {
+        const int base = ((int)(c.pk & LM) + lx) + a.Sx * (int)(c.pk >> 16);
+#pragma unroll
+        for (int ly = 0; ly < W; ++ly) {
+          const C v = tile[base + a.Sx * ly];
+          ar = fma(c.w2[ly], v.x, ar);
+          ai = fma(c.w2[ly], v.y, ai);
+        }
+        ar *= c.w1;
+        ai *= c.w1;
+      } else {
+        const C v = tile[(int)c.pk + lx];
+        ar = c.w1 * v.x;
+        ai = c.w1 * v.y;
+      }
+    }
+    ar = group_sum<G>(ar);
+    ai = group_sum<G>(ai);
+    if (lx == 0 && on) fhat[(long long)c.pj * a.fst] = C{ar * osc, ai * osc};
   }
 }
 

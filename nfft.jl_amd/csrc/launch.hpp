@@ -84,8 +84,8 @@ hipError_t launch_inv_perm(const int* perm, int* iperm, long long n, hipStream_t
 hipError_t launch_gather_nodes(bool dbl, const void* in, long long is, const int* idx, void* out, long long os,
                                long long n, hipStream_t s, int s0, int nsl);
 
-// LDS bytes of a tile kernel.
-size_t tile_lds_bytes(int D, bool dbl, int W, int tileElems);
+// LDS bytes of a 1-D or 2-D tile kernel.
+size_t tile_lds_bytes(bool dbl, int tileElems);
 
 // Tile kernels (D = 1, 2, 3).  grid = 8 * ceil(nitems / 8) workgroups of NT.
 hipError_t launch_tile(int D, bool spread, bool dbl, int W, int NT, const KArgs& a, size_t lds,

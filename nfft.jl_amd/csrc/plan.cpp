@@ -434,9 +434,10 @@ struct nfftm_plan_s {
   int sl0 = 0, sln = 1, gcap = 1, scap = 1;
   // 3-D scratch slots in halo/interior block layout: halos (m - 1, m cells)
   // no wider than any tile, a partial last one included
+  // (2-D: the fold by tiles)
   bool blocked3() const {
-    if (D != 3 || !tiled) return false;
-    for (int d = 0; d < 3; ++d)
+    if (D < 2 || !tiled) return false;
+    for (int d = 0; d < D; ++d)
       if (T[d] < m || Nt[d] - (ntiles[d] - 1) * T[d] < m) return false;
     return true;
   }
@@ -620,8 +621,7 @@ struct nfftm_plan_s {
     a.tileElems = tileElems;
     a.padCells = Pd[0] * Pd[1] * Pd[2];
     a.divP0 = make_fastdiv((uint32_t)Pd[0]);
-    a.divP1 = make_fastdiv((uint32_t)Pd[1]);
-    a.divNtx = make_fastdiv((uint32_t)std::max<i64>(1, Nt[0]));
+    a.divT0 = make_fastdiv((uint32_t)std::max(1, T[0]));
     a.lut = d_lut.p;
     a.scale = LUTSize / m;
     a.poly = d_poly.p;
@@ -827,7 +827,7 @@ bool set_tile_shape(nfftm_plan_s& p, int t) {
   if (D >= 2 && Pd[0] % 16 == 7) Sx = Pd[0] + 1;
   const int Sxy = Sx * (D >= 2 ? Pd[1] : 1);
   const int te = Sxy;
-  const size_t bytes = tile_lds_bytes(D, p.dbl(), W, te);
+  const size_t bytes = tile_lds_bytes(p.dbl(), te);
   for (int d = 0; d < 3; ++d) {
     p.T[d] = D > d ? T[d] : 1;
     p.Pd[d] = D > d ? Pd[d] : 1;
@@ -1835,6 +1835,11 @@ int batch_build(nfftm_batch_s& b, const nfftm_plan* plans, const int* ntrans, in
     const i64 rows = p.P / p.N[0], CR = std::max<i64>(1, 1024 / p.N[0]);
     for (i64 r0 = 0; r0 < rows; r0 += CR) dect.push_back(int4{s, (int)r0, (int)std::min(rows, r0 + CR), 0});
     if (p.D == 2) {
+      if (p.blocked3()) {
+        for (int t = 0; t < p.ntiles[0] * p.ntiles[1]; ++t)
+          for (int c = 0; c < p.T[0] * p.T[1]; c += 256) fold[1].push_back(int4{s, c, t, 0});
+        continue;
+      }
       const i64 CF = std::max<i64>(1, 1024 / p.Nt[0]);
       for (i64 r0 = 0; r0 < p.Nt[1]; r0 += CF)
         fold[1].push_back(int4{s, (int)r0, (int)std::min<i64>(p.Nt[1], r0 + CF), 0});
