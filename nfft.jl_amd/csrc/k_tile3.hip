@@ -95,6 +95,20 @@ struct Blocks3 {
   }
 };
 
+// Offsets of the 27 blocks as a table.
+template <int W, int T, int TZ>
+struct BlockTable {
+  struct Tab {
+    int off[27];
+  };
+  static constexpr __host__ __device__ Tab make() {
+    Tab t{};
+    for (int b = 0; b < 27; ++b) t.off[b] = Blocks3<W, T, TZ>::off(b);
+    return t;
+  }
+  static constexpr Tab tab = make();
+};
+
 // Compile-time loop: f(std::integral_constant<int, I>) for I in [I0, N).
 template <int I0, int N, typename F>
 __device__ __forceinline__ void static_for(F&& f) {
@@ -276,15 +290,14 @@ void k_interp3(KArgs a, const typename cpx<R>::T* __restrict__ grid,
   }
 }
 
-// Spreading in FP32: lanes over the (x, y) columns of a node's footprint,
-// walking z, one LDS atomic per tap on packed 32+32-bit fixed point with a
-// per-item scale from a strict bound; the padded tile goes to the item's
-// scratch slot.
-template <int W, int NT, int V>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(V == 1 && W <= 12 ? NT / 128 : 1)))
-void k_spread3(KArgs a, const float2* __restrict__ fhat) {
-  using R = float;
-  using C = float2;
+// Spreading: lanes over the (x, y) columns of a node's footprint, walking z,
+// one LDS atomic per tap (FP32: packed 32+32-bit fixed point with a per-item
+// scale from a strict bound; FP64: two FP64 planes, W <= 8); the padded tile
+// goes to the item's scratch slot.
+template <typename R, int W, int NT, int V>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(V == 1 && W <= (sizeof(R) == 4 ? 12 : 8) ? NT / 128 : 1)))
+void k_spread3(KArgs a, const typename cpx<R>::T* __restrict__ fhat) {
+  using C = typename cpx<R>::T;
   using G = Geo3<R, W, V>;
   constexpr int NW = NT / 64;
   extern __shared__ __align__(16) char smem[];
@@ -314,9 +327,9 @@ void k_spread3(KArgs a, const float2* __restrict__ fhat) {
   // clear the tile while the gathers are in flight
   for (int i = threadIdx.x; i < (int)(G::TILE_BYTES / 16); i += NT) ((uint4*)tile)[i] = make_uint4(0, 0, 0, 0);
 
-  // fixed-point scale s = 2^(30 - e), B = sum_j |f_j|_inf * wmaxD < 2^e
+  // FP32: fixed-point scale s = 2^(30 - e), B = sum_j |f_j|_inf * wmaxD < 2^e
   R fscale = 1, inv = 1;
-  {
+  if (sizeof(R) == 4) {
     R part = 0;
 #pragma unroll
     for (int h = 0; h < HPT; ++h) part += fmax(fabs(hre[h]), fabs(him[h]));
@@ -388,15 +401,26 @@ void k_spread3(KArgs a, const float2* __restrict__ fhat) {
           const R wxy = w[lx] * w[W + ly];
           const R vr = f.x * wxy, vi = f.y * wxy;
           const int base = cell + lx + G::SX * ly;
-          unsigned long long* tl = (unsigned long long*)tile + base;
+          if constexpr (sizeof(R) == 4) {
+            unsigned long long* tl = (unsigned long long*)tile + base;
 #pragma unroll
-          for (int lz = 0; lz < W; ++lz) {
-            int re, im;
-            asm volatile("v_cvt_rpi_i32_f32 %0, %1" : "=v"(re) : "v"((float)(vr * w3[lz])));
-            asm volatile("v_cvt_rpi_i32_f32 %0, %1" : "=v"(im) : "v"((float)(vi * w3[lz])));
-            const unsigned long long term =
-                ((unsigned long long)(unsigned)(im + (re >> 31)) << 32) | (unsigned)re;
-            __hip_atomic_fetch_add(tl + G::SXY * lz, term, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            for (int lz = 0; lz < W; ++lz) {
+              int re, im;
+              asm volatile("v_cvt_rpi_i32_f32 %0, %1" : "=v"(re) : "v"((float)(vr * w3[lz])));
+              asm volatile("v_cvt_rpi_i32_f32 %0, %1" : "=v"(im) : "v"((float)(vi * w3[lz])));
+              const unsigned long long term =
+                  ((unsigned long long)(unsigned)(im + (re >> 31)) << 32) | (unsigned)re;
+              __hip_atomic_fetch_add(tl + G::SXY * lz, term, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+          } else {
+            double* tr = (double*)tile + base;
+#pragma unroll
+            for (int lz = 0; lz < W; ++lz) {
+              __hip_atomic_fetch_add(tr + G::SXY * lz, (double)(vr * w3[lz]), __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_WORKGROUP);
+              __hip_atomic_fetch_add(tr + G::CELLS + G::SXY * lz, (double)(vi * w3[lz]), __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
           }
         }
       }
@@ -440,209 +464,82 @@ void k_spread3(KArgs a, const float2* __restrict__ fhat) {
   }
 }
 
-
 // Spreading in FP64 on the matrix cores.  The padded tile is a contraction
 // over the item's nodes j,
 //   tile[z, (y, x)] = sum_j wz_j[z] * (wy_j[y] wx_j[x] f_j),
 // with the weights zero outside a node's footprint: v_mfma_f64_16x16x4 with
 // 16 z rows, 16 columns of the flattened (y, x) plane and 4 nodes per
-// instruction, once for the real and once for the imaginary part.  The tile
-// lives in the accumulators (wavefront w holds the column tiles w, w + NW,
-// ...), so there is no LDS tile to clear, no atomic, and a fixed order of
-// the sums within a batch order.
+// instruction, once for the real and once for the imaginary part.
 //
-// A batch of nodes is sorted in LDS by the z rows its footprint reaches (one
-// or two row tiles) and by y, so that four neighbours share their rows: only
-// the column tiles of those rows (W + 1 or so of T + W - 1) are multiplied.
-// The cost per node is about (W + 2) P / 16 column tiles x 2 x 16 cycles / 4
-// (m = 5: 156 cycles per CU; m = 4: 75), against ceil(W^2 / 64) W 2 LDS adds
-// of 9 cycles or more (400; 160).
-// MFMA_NOTE
-template <int W, int NT, int V>
+// A batch of nodes is staged in LDS with its weights zero-padded to the whole
+// padded range (so that the products need no bounds), sorted by the row
+// tiles it reaches and by y.  A wavefront takes one 16 x 16 tile at a time:
+// the nodes that reach the tile's rows are one run of the sorted list (two
+// for the first of two row tiles), so only about W + 1 of the T + W - 1 rows of
+// y are multiplied; the tile is then stored to the slot while the next one is
+// computed.  One tile's accumulators (16 registers) leave room for two
+// workgroups of 1024 threads per CU, one's staging beside the other's products.
+// On a 96^3 image with 10^6 nodes, m = 5: 565 us, of which the products are 235
+// us of the matrix cores (two LDS adds per tap: 1241 us; accumulators for the
+// whole padded tile, one workgroup per CU: 777; 512 threads: 609).
+// Per node (W + 2) P / 16 tiles x 2 x 16 cycles / 4 of the matrix cores (m = 5:
+// 156 cycles per CU; m = 4: 75) against ceil(W^2 / 64) W 2 LDS adds of 9 cycles
+// or more (400; 160).  Up to W = 8 the adds stay ahead on thinly sampled
+// grids (64^3 image, 2 10^4 nodes, m = 4: 47 us against 70; 2 10^5 nodes on
+// 96^3, m = 3: 131 against 158) and near on dense ones (128^3, 2^21 nodes,
+// m = 4: 1122 against 1012); from W = 10 on the products are ahead on both (m =
+// 5: 2 10^4 nodes 97 against 52, 10^6 nodes 1081 against 579; m = 6: 639
+// against 292).
+template <int W, int V>
 struct Mf3 {
   using G = Geo3<double, W, V>;
-  static constexpr int NW = NT / 64;
-  static constexpr int NCOL = G::P * G::P, NTC = (NCOL + 15) / 16, TPW = (NTC + NW - 1) / NW;
-  static constexpr int MT = (G::PZ + 15) / 16;
-  static_assert(MT <= 2, "padded z rows");
-  static constexpr int RS = 3 * W + 1;  // doubles of a node's weights in LDS (odd: spread over the banks)
-  static constexpr size_t bytes(int nb) { return (size_t)nb * (RS * 8 + 16 + 8) + (nb / 4) * 4 + 64 * 4 + 32 * 4 + 64; }
-  static constexpr int NB = bytes(256) <= 81920 ? 256 : 128;
-  static constexpr size_t W_OFF = 0, F_OFF = W_OFF + (size_t)NB * RS * 8, C_OFF = F_OFF + (size_t)NB * 16,
-                          G_OFF = C_OFF + (size_t)NB * 8, H_OFF = G_OFF + (size_t)NB, O_OFF = H_OFF + 64 * 4,
-                          LDS = O_OFF + 32 * 4;
-  static_assert(LDS <= bytes(NB) && NB <= NT && MT * G::T <= 32, "FP64 spreading layout");
+  static constexpr int NT = 1024, NW = NT / 64;
+  static constexpr int NCOL = G::P * G::P, NTC = (NCOL + 15) / 16;  // columns and column tiles
+  static constexpr int MT = (G::PZ + 15) / 16;                     // row tiles
+  static constexpr int RS = (2 * G::P + G::PZ) | 1;  // doubles per node: x, y, z weights (odd: spread over the banks)
+  static_assert(MT <= 2 && MT * G::T < 63, "FP64 spreading");
+  // LDS of batches of nb nodes (and a zero one): weights (and what the last
+  // row tile reads past them), values, per node its sorted position and cell
+  static constexpr size_t f_off(int nb) { return ((size_t)(nb + 1) * RS + 32) * 8 / 16 * 16 + 16; }
+  static constexpr size_t p_off(int nb) { return f_off(nb) + (size_t)(nb + 1) * 16; }
+  static constexpr size_t h_off(int nb) { return p_off(nb) + (size_t)nb * 8; }
+  static constexpr size_t lds(int nb) { return h_off(nb) + 64 * 4; }
+  static constexpr int fit(size_t cap) {
+    int nb = 512;
+    while (lds(nb) > cap) nb -= 16;
+    return nb;
+  }
+  // two workgroups per CU, or one where the tiles hold more nodes than that
+  // (a second batch adds to the slot instead of storing it)
+  static constexpr int NB2 = fit(81920), NB1 = fit(163840);
+  static_assert(NB2 >= 64, "batch");
 };
 
-template <int W, int NT, int V>
-__global__ __launch_bounds__(NT) void k_spread3d(KArgs a, const double2* __restrict__ fhat) {
-  using M = Mf3<W, NT, V>;
+template <int W, int V>
+__global__ __launch_bounds__((Mf3<W, V>::NT)) __attribute__((amdgpu_waves_per_eu(8)))
+void k_spread3d(KArgs a, const double2* __restrict__ fhat, int NB) {
+  using M = Mf3<W, V>;
   using G = typename M::G;
   typedef double d4 __attribute__((ext_vector_type(4)));
-  constexpr int P = G::P, NW = M::NW, RS = M::RS, NB = M::NB, MT = M::MT, TPW = M::TPW, RB = G::RB;
-  constexpr int NU = 3 * W / 2;                          // 16-byte words of a node's weights
-  constexpr int PER = (NB * NU + NT - 1) / NT;
+  constexpr int P = G::P, T = G::T, NW = M::NW, NT = M::NT, RS = M::RS, MT = M::MT, RB = G::RB, m = W / 2;
+  constexpr int NU = 3 * W / 2;  // 16-byte words of a node's weights
+  constexpr int CP = 3;          // of them in flight per thread
   extern __shared__ __align__(16) char smem[];
-  double* lw = (double*)(smem + M::W_OFF);               // weights, node by node
-  double2* sf = (double2*)(smem + M::F_OFF);             // sorted: values
-  int2* sc = (int2*)(smem + M::C_OFF);                   // sorted: cell (x, y << 8, z << 16), first weight
-  int* gr = (int*)(smem + M::G_OFF);                     // per four nodes: first, last column tile, second row tile
-  int* hist = (int*)(smem + M::H_OFF);                   // buckets (row tiles, y), then their starts
-  int* boff = (int*)(smem + M::O_OFF);                   // block offsets of the slot
+  double* lw = (double*)smem;
+  double2* sf = (double2*)(smem + M::f_off(NB));
+  int2* pos = (int2*)(smem + M::p_off(NB));  // first double of the node's weights, cell (x, y << 8, z << 16)
+  int* hist = (int*)(smem + M::h_off(NB));   // nodes per (row tiles, y), then their starts; [63]: all
   const int item = xcd_item(a.nitems);
   if (item >= a.nitems) return;
   const int4 it = a.items[item];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int c16 = lane & 15, k4 = lane >> 4;
-
-  // the lane's column of each of its tiles
-  int xi[TPW], yi[TPW];
-  d4 acc[TPW][2][MT];
-#pragma unroll
-  for (int i = 0; i < TPW; ++i) {
-    const int q = (wave + i * NW) * 16 + c16;
-    yi[i] = q / P;
-    xi[i] = q - yi[i] * P;
-#pragma unroll
-    for (int r = 0; r < MT; ++r) acc[i][0][r] = acc[i][1][r] = d4{0, 0, 0, 0};
-  }
-  if (tid < 27) {
-    using B = Blocks3<W, G::T, G::TZ>;
-    int o = 0;
-    if (tid != 13) {
-      o = B::size(13);
-      for (int q = 0; q < tid; ++q) o += q == 13 ? 0 : B::size(q);
-    }
-    boff[tid] = o;
-  }
-
-  // one batch ahead: weights (16-byte words of the records), and the cell and
-  // value of node b0 + tid
-  uint4 rw[PER];
-  int loc = 0;
-  double2 val{0, 0};
-  auto fetch = [&](int b0) {
-    const int nb = min(NB, it.z - b0);
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int i = tid + u * NT, n = i / NU;
-      if (n < nb) rw[u] = ((const uint4*)(a.rec + (size_t)(b0 + n) * RB))[i - n * NU];
-    }
-    if (tid < nb) {
-      const int2 q = *(const int2*)(a.rec + (size_t)(b0 + tid) * RB + NodeRec<double, 3, W>::WBYTES);
-      loc = q.x;
-      val = fhat[(long long)q.y * a.fst];
-    }
-  };
-  fetch(it.y);
-  for (int b0 = it.y; b0 < it.z; b0 += NB) {
-    const int nb = min(NB, it.z - b0), ng = (nb + 3) >> 2;
-    __syncthreads();  // the batch before is done with the LDS
-    if (tid < 64) hist[tid] = 0;
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      const int i = tid + u * NT, n = i / NU;
-      if (n < nb) {
-        double* d = lw + n * RS + 2 * (i - n * NU);
-        d[0] = __hiloint2double((int)rw[u].y, (int)rw[u].x);
-        d[1] = __hiloint2double((int)rw[u].w, (int)rw[u].z);
-      }
-    }
-    __syncthreads();
-    // sort: bucket = (reaches the second row tile, y)
-    int key = 0, rank = 0, cell = 0;
-    if (tid < nb) {
-      const int cz = loc / G::SXY, r = loc - cz * G::SXY, cy = r / G::SX, cx = r - cy * G::SX;
-      cell = cx | cy << 8 | cz << 16;
-      key = (MT == 2 && cz + W > 16 ? G::T : 0) + cy;
-      rank = __hip_atomic_fetch_add(&hist[key], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    }
-    __syncthreads();
-    if (tid < 64) {
-      const int h = hist[tid];
-      int s = h;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int t = __shfl_up(s, o);
-        if (lane >= o) s += t;
-      }
-      hist[tid] = s - h;
-    }
-    __syncthreads();
-    if (tid < nb) {
-      const int d = hist[key] + rank;
-      sc[d] = int2{cell, tid * RS};
-      sf[d] = double2{val.x * a.oscale, val.y * a.oscale};
-    } else if (tid < 4 * ng) {  // up to a whole group: value 0 at node 0's weights
-      sc[tid] = int2{0, 0};
-      sf[tid] = double2{0, 0};
-    }
-    __syncthreads();
-    if (tid < ng) {
-      int lo = 1 << 20, hi = 0, z2 = 0;
-#pragma unroll
-      for (int n = 0; n < 4; ++n) {
-        if (4 * tid + n < nb) {
-          const int cl = sc[4 * tid + n].x, cy = cl >> 8 & 255;
-          lo = min(lo, cy);
-          hi = max(hi, cy);
-          z2 |= MT == 2 && (cl >> 16) + W > 16;
-        }
-      }
-      gr[tid] = lo * P / 16 | ((hi + W) * P - 1) / 16 << 8 | z2 << 16;
-    }
-    if (b0 + NB < it.z) fetch(b0 + NB);
-    __syncthreads();
-
-    for (int g = 0; g < ng; ++g) {
-      const int range = __builtin_amdgcn_readfirstlane(gr[g]);
-      const int t0 = range & 255, t1 = range >> 8 & 255;
-      const bool two = MT == 2 && range >> 16;
-      // a column tile of this wavefront in [t0, t1]?
-      if (wave + (t0 - wave + NW - 1 + NW * 64) / NW * NW - NW * 64 > t1) continue;
-      const int2 s = sc[4 * g + k4];
-      const double2 f = sf[4 * g + k4];
-      const int cx = s.x & 255, cy = s.x >> 8 & 255, cz = s.x >> 16;
-      const double* w = lw + s.y;
-      double az[MT];
-#pragma unroll
-      for (int r = 0; r < MT; ++r) {
-        const int z = c16 + 16 * r - cz;
-        const bool in = (unsigned)z < (unsigned)W;
-        const double v = w[2 * W + (in ? z : 0)];
-        az[r] = in ? v : 0.0;
-      }
-#pragma unroll
-      for (int i = 0; i < TPW; ++i) {
-        const int t = wave + i * NW;
-        if (t < t0 || t > t1) continue;
-        const int x = xi[i] - cx, y = yi[i] - cy;
-        const bool in = (unsigned)x < (unsigned)W && (unsigned)y < (unsigned)W;
-        const double wx = w[in ? x : 0], wy = w[W + (in ? y : 0)];
-        const double wxy = in ? wx * wy : 0.0;
-        const double br = wxy * f.x, bi = wxy * f.y;
-        acc[i][0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(az[0], br, acc[i][0][0], 0, 0, 0);
-        acc[i][1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(az[0], bi, acc[i][1][0], 0, 0, 0);
-        if constexpr (MT == 2) {
-          if (two) {
-            acc[i][0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(az[1], br, acc[i][0][1], 0, 0, 0);
-            acc[i][1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(az[1], bi, acc[i][1][1], 0, 0, 0);
-          }
-        }
-      }
-    }
-  }
-  if (it.y >= it.z) __syncthreads();
-
-  // accumulators -> the item's scratch slot: element (row k4 + 4 e, column
-  // c16) of each 16 x 16 tile
   double2* out = (double2*)a.scratch + (size_t)item * G::SLOT;
-  constexpr int m = W / 2;
   int h[3];  // end of the tile's own cells in the padded range
   {
     const int tx = it.x % a.ntiles[0], q = it.x / a.ntiles[0], ty = q % a.ntiles[1], tz = q / a.ntiles[1];
-    h[0] = m - 1 + min(G::T, a.Nt[0] - tx * G::T);
-    h[1] = m - 1 + min(G::T, a.Nt[1] - ty * G::T);
+    h[0] = m - 1 + min(T, a.Nt[0] - tx * T);
+    h[1] = m - 1 + min(T, a.Nt[1] - ty * T);
     h[2] = m - 1 + min(G::TZ, a.Nt[2] - tz * G::TZ);
   }
   auto part = [&](int v, int e, int t, int* b, int* l, int* ext) {
@@ -650,26 +547,113 @@ __global__ __launch_bounds__(NT) void k_spread3d(KArgs a, const double2* __restr
     *l = *b == 0 ? v : *b == 1 ? v - (m - 1) : v - e;
     *ext = *b == 0 ? m - 1 : *b == 1 ? t : m;
   };
+
+  for (int b0 = it.y; b0 < it.z; b0 += NB) {
+    const int nb = min(NB, it.z - b0);
+    int loc = 0;
+    double2 val{0, 0};
+    if (tid < nb) {
+      const int2 q = *(const int2*)(a.rec + (size_t)(b0 + tid) * RB + NodeRec<double, 3, W>::WBYTES);
+      loc = q.x;
+      val = fhat[(long long)q.y * a.fst];
+    }
+    // the first CP words of weights per thread, in flight during the sort
+    uint4 rw[CP];
+    auto words = [&](int i0) {
 #pragma unroll
-  for (int i = 0; i < TPW; ++i) {
-    const int x = xi[i], y = yi[i];
-    if (y >= P) continue;
-    int bx, by, lx, ly, ex, ey;
-    part(x, h[0], G::T, &bx, &lx, &ex);
-    part(y, h[1], G::T, &by, &ly, &ey);
-    const bool in = x < h[0] + m && y < h[1] + m;
+      for (int u = 0; u < CP; ++u) {
+        const int i = min(i0 + u * NT, nb * NU - 1), n = i / NU;
+        rw[u] = *(const uint4*)(a.rec + (size_t)(b0 + n) * RB + 16 * (i - n * NU));
+      }
+    };
+    words(tid);
+    __syncthreads();  // the batch before is done with the LDS
+    if (tid < 64) hist[tid] = 0;
+    for (int i = tid; i < ((nb + 1) * RS + 1) / 2; i += NT) ((double2*)lw)[i] = double2{0, 0};
+    __syncthreads();
+    // sort by (reaches the second row tile, y)
+    int key = 0, rank = 0, cell = 0;
+    if (tid < nb) {
+      const int cz = loc / G::SXY, r = loc - cz * G::SXY, cy = r / G::SX, cx = r - cy * G::SX;
+      cell = cx | cy << 8 | cz << 16;
+      key = (MT == 2 && cz + W > 16 ? T : 0) + cy;
+      rank = __hip_atomic_fetch_add(&hist[key], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    __syncthreads();
+    if (tid < 64) {
+      const int c = hist[tid];
+      int s = c;
 #pragma unroll
-    for (int r = 0; r < MT; ++r) {
+      for (int o = 1; o < 64; o <<= 1) {
+        const int t = __shfl_up(s, o);
+        if (lane >= o) s += t;
+      }
+      hist[tid] = s - c;
+    }
+    __syncthreads();
+    if (tid < nb) {
+      const int d = hist[key] + rank;
+      pos[tid] = int2{d * RS, cell};
+      sf[d] = double2{val.x * a.oscale, val.y * a.oscale};
+    }
+    if (tid == 0) sf[nb] = double2{0, 0};
+    __syncthreads();
+    // weights to their places in the padded ranges
+    for (int i0 = tid; i0 < nb * NU; i0 += CP * NT) {
+      if (i0 > tid) words(i0);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int z = 16 * r + 4 * e + k4;
-        const double2 v{acc[i][0][r][e], acc[i][1][r][e]};
+      for (int u = 0; u < CP; ++u) {
+        const int i = min(i0 + u * NT, nb * NU - 1), n = i / NU, w = i - n * NU, d = w / m;
+        const int2 p = pos[n];
+        double* q = lw + p.x + d * P + (p.y >> 8 * d & 255) + 2 * (w - d * m);
+        q[0] = __hiloint2double((int)rw[u].y, (int)rw[u].x);
+        q[1] = __hiloint2double((int)rw[u].w, (int)rw[u].z);
+      }
+    }
+    __syncthreads();
+
+    for (int j = wave; j < M::NTC * MT; j += NW) {
+      const int rt = j >= M::NTC ? 1 : 0, t = j - rt * M::NTC;
+      const int q = 16 * t + c16, y = q / P, x = q - y * P, z0 = 16 * rt;
+      // cells (y) whose footprint reaches the tile's rows of y
+      const int lo = max(0, 16 * t / P - W + 1), hi = min(T - 1, (16 * t + 15) / P);
+      d4 re{0, 0, 0, 0}, im{0, 0, 0, 0};
+      for (int c = rt; c < MT; ++c) {
+        const int s = __builtin_amdgcn_readfirstlane(hist[c * T + lo]);
+        const int e = __builtin_amdgcn_readfirstlane(hist[c * T + hi + 1]);
+        for (int n = s; n < e; n += 4) {
+          const int i = n + k4 < e ? n + k4 : nb;  // nb: the zero node
+          const double* w = lw + i * RS;
+          const double2 f = sf[i];
+          const double wz = w[2 * P + z0 + c16], wxy = w[x] * w[P + y];
+          re = __builtin_amdgcn_mfma_f64_16x16x4f64(wz, wxy * f.x, re, 0, 0, 0);
+          im = __builtin_amdgcn_mfma_f64_16x16x4f64(wz, wxy * f.y, im, 0, 0, 0);
+        }
+      }
+      // element (row k4 + 4 i, column c16) -> the item's scratch slot
+      int bx, by, lx, ly, ex, ey;
+      part(x, h[0], T, &bx, &lx, &ex);
+      part(y, h[1], T, &by, &ly, &ey);
+      const bool in = y < P && (!a.blocked3 || (x < h[0] + m && y < h[1] + m));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int z = z0 + 4 * i + k4;
+        int o = x + P * (y + P * z);
+        bool st = in && z < G::PZ;
         if (a.blocked3) {
           int bz, lz, ez;
           part(z, h[2], G::TZ, &bz, &lz, &ez);
-          if (in && z < h[2] + m) out[boff[bx + 3 * by + 9 * bz] + lx + ex * (lz + ez * ly)] = v;
-        } else if (z < G::PZ) {
-          out[x + P * (y + P * z)] = v;
+          st = in && z < h[2] + m;
+          o = BlockTable<W, T, G::TZ>::tab.off[bx + 3 * by + 9 * (st ? bz : 0)] + lx + ex * (lz + ez * ly);
+        }
+        if (st) {
+          double2 v{re[i], im[i]};
+          if (b0 > it.y) {
+            const double2 p = out[o];
+            v.x += p.x;
+            v.y += p.y;
+          }
+          out[o] = v;
         }
       }
     }
@@ -1010,17 +994,19 @@ static hipError_t go3(bool spread, int NT, const KArgs& a, hipStream_t s, const 
     const int nblk = 8 * ((a.nitems + 7) / 8);
     const int lds = (int)G::LDS;
     (void)out;
-    if constexpr (sizeof(R) == 8) {
+    if constexpr (sizeof(R) == 8 && W >= 10) {
       if (spread) {
-        const int ls = (int)(NT == 1024 ? Mf3<W, 1024, V>::LDS : Mf3<W, 512, V>::LDS);
-        auto k = NT == 1024 ? k_spread3d<W, 1024, V> : k_spread3d<W, 512, V>;
+        using M = Mf3<W, V>;
+        auto k = k_spread3d<W, V>;
+        const int nb = (long long)a.M > (long long)a.nitems * M::NB2 ? M::NB1 : M::NB2;
+        const int ls = (int)M::lds(nb);
         if (hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, ls) != hipSuccess)
           return hipErrorInvalidConfiguration;
-        hipLaunchKernelGGL(k, dim3(nblk), dim3(NT), ls, s, a, (const C*)in);
+        hipLaunchKernelGGL(k, dim3(nblk), dim3(M::NT), ls, s, a, (const C*)in, nb);
         return hipGetLastError();
       }
     } else if (spread) {
-      auto k = NT == 1024 ? k_spread3<W, 1024, V> : k_spread3<W, 512, V>;
+      auto k = NT == 1024 ? k_spread3<R, W, 1024, V> : k_spread3<R, W, 512, V>;
       if (hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
         return hipErrorInvalidConfiguration;
       hipLaunchKernelGGL(k, dim3(nblk), dim3(NT), lds, s, a, (const C*)in);

@@ -1,9 +1,11 @@
-"""FP64 3-D spreading on the matrix cores (k_spread3d) against the oracle.
+"""FP64 3-D spreading against the oracle: on the matrix cores from 2m = 10 on
+(k_spread3d: two row tiles along z, whole and partial column tiles), by LDS
+adds below.
 
-Every stencil width 2m = 2 .. 16 (one or two row tiles along z, whole and
-partial column tiles), both tile geometries and both workgroup sizes, nodes
-that fill groups of four exactly, leave one over, or share one cell, tiles of
-one node, items of several batches and several items; FP64 rel-l2 <= 1e-12.
+Every stencil width 2m = 2 .. 16, both tile geometries and both workgroup
+sizes, nodes that fill groups of four exactly, leave one over, or share one
+cell, tiles of one node, items of several batches and several items; FP64
+rel-l2 <= 1e-12.
 """
 import numpy as np
 import pytest
@@ -52,5 +54,5 @@ def test_counts(M):
     rng = np.random.default_rng(M)
     for spread in (0.0, 0.04):
         k = 0.11 + spread * (rng.random((3, M)) - 0.5)
-        for m in (4, 5):
+        for m in (4, 5, 6):
             check(k, (24, 24, 24), m)
