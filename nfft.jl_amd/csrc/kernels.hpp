@@ -127,6 +127,13 @@ struct KArgs {
   // slot 0, the plan's grid), its scratch slots follow those of s - 1
   int s0, nsl;
   long long Bsl, Q;
+  // density compensation on 2-D tiled plans, fused (null otherwise): k_fold2
+  // divides the grid by gdiv[0]; interpolation, instead of storing its
+  // result, divides the real weights wdiv of the nodes by its real part over
+  // gdiv[0] and flags results that are not positive
+  const double* gdiv;
+  void* wdiv;
+  int* wbad;
 };
 
 // (Bsl < 2^31; slice 0, the only one of an ordinary plan, needs no division)
@@ -784,6 +791,11 @@ __device__ __forceinline__ void fold2_point(const KArgs& a, const typename cpx<R
       }
     }
   }
+  if (a.gdiv) {
+    const R d = (R)a.gdiv[0];
+    sr /= d;
+    si /= d;
+  }
   if (in) grid[(long long)y * a.Nt[0] + x] = C{sr, si};
 }
 
@@ -859,11 +871,13 @@ __device__ __forceinline__ void interp_tile_item(const KArgs& a, int item,
   }
   __syncthreads();
 
-  const R osc = (R)a.oscale;
+  const R osc = (R)a.oscale, gd = D == 2 && a.wdiv ? (R)a.gdiv[0] : (R)1;
   for (int n0 = it.y + wave * NPW; n0 < it.z; n0 += NW * NPW) {
     const int n = n0 + slot;
     const bool on = n < it.z;
     const NodeTaps<R, D, W> c = nx;
+    R wold = 0;  // the weight to be divided, in flight during the taps
+    if (D == 2 && a.wdiv && lx == 0 && on) wold = ((const C*)a.wdiv)[c.pj].x;
     const int m = n + NW * NPW;
     nx.load(a.rec, m < it.z ? m : it.y, lw);
     R ar = 0, ai = 0;
@@ -886,7 +900,15 @@ __device__ __forceinline__ void interp_tile_item(const KArgs& a, int item,
     }
     ar = group_sum<G>(ar);
     ai = group_sum<G>(ai);
-    if (lx == 0 && on) fhat[(long long)c.pj * a.fst] = C{ar * osc, ai * osc};
+    if (lx == 0 && on) {
+      if (D == 2 && a.wdiv) {
+        const R t = ar * osc / gd;
+        if (!(t > (R)0)) a.wbad[0] = 1;
+        ((C*)a.wdiv)[c.pj] = C{wold / t, (R)0};
+      } else {
+        fhat[(long long)c.pj * a.fst] = C{ar * osc, ai * osc};
+      }
+    }
   }
 }
 

@@ -1205,8 +1205,21 @@ bool fused_fold(const nfftm_plan_s& p) {
          launch_fold_fft3(p.dbl(), p.W, p.kargs(), p.fargs(), nullptr, nullptr, true) == hipSuccess;
 }
 
-int run_conv(nfftm_plan_s& p, bool spread, const void* in, void* out, bool standalone = false, bool fold = true) {
+// sdc: the fused steps of density compensation (KArgs gdiv, wdiv, wbad).
+struct SdcFuse {
+  const double* gdiv;
+  void* wdiv;
+  int* wbad;
+};
+
+int run_conv(nfftm_plan_s& p, bool spread, const void* in, void* out, bool standalone = false, bool fold = true,
+             const SdcFuse* sdc = nullptr) {
   KArgs a = p.kargs();
+  if (sdc) {
+    a.gdiv = sdc->gdiv;
+    a.wdiv = sdc->wdiv;
+    a.wbad = sdc->wbad;
+  }
   if (standalone) a.oscale = std::pow(p.wscale, -(double)p.D);
   hipError_t e;
   if (spread && !p.tiled) {
@@ -2532,10 +2545,21 @@ int sdc_impl(nfftm_plan_s* p, int iters, void* weights, int scale, const SdcWork
   HIPCHK(launch_fill0(w.bad, sizeof(int), s));
   HIPCHK(launch_real_to_cpx(dbl, weights, w.wc, M, s));
   // sdc!(p, iters, weights, weights_tmp, workg), samplingDensity.jl:93-118
+  // 2-D tiled plans: the division by the first maximum is made by the fold
+  // (from the second iteration on) and the update of the weights by the
+  // interpolation, with the same operations on each value; two passes over
+  // the grid and the nodes fewer per iteration (512^2 points, 2 10^5 nodes:
+  // 4 + 4 of 39 us)
+  const bool fused = p->tiled && p->D == 2 && p->blocked3();
+  const SdcFuse fdiv{w.sc, nullptr, nullptr}, fupd{w.sc, w.wc, w.bad};
   for (int i = 0; i < iters; ++i) {
-    if (int rc = run_conv(*p, true, w.wc, p->d_grid.p, true)) return rc;
+    if (int rc = run_conv(*p, true, w.wc, p->d_grid.p, true, true, fused && i > 0 ? &fdiv : nullptr)) return rc;
     if (i == 0) HIPCHK(launch_reduce(dbl, RED_MAX_RE, p->d_grid.p, p->Q, part, w.sc, s));
-    HIPCHK(launch_div_scalar(dbl, p->d_grid.p, p->Q, w.sc, s));
+    if (!fused || i == 0) HIPCHK(launch_div_scalar(dbl, p->d_grid.p, p->Q, w.sc, s));
+    if (fused) {
+      if (int rc = run_conv(*p, false, p->d_grid.p, w.wt, true, true, &fupd)) return rc;
+      continue;
+    }
     if (int rc = run_conv(*p, false, p->d_grid.p, w.wt, true)) return rc;
     HIPCHK(launch_sdc_update(dbl, w.wc, w.wt, M, w.sc, w.bad, s));
   }
