@@ -401,6 +401,48 @@ __global__ __launch_bounds__(MixBlock<R>::NT) void k_mix_col(MixArgs a, typename
       });
 }
 
+// The strided pass of the last dimension in both directions with a product
+// between (the Toeplitz embedding: FFT, eigenvalues, inverse FFT): the line
+// stays in LDS, where separate passes would write, multiply and read the grid
+// once more each.  The transformed line goes to a second LDS area, since other
+// threads still read the first one.
+template <typename R>
+__global__ __launch_bounds__(MixBlock<R>::NT) void k_mix_mul(MixArgs a, typename cpx<R>::T* __restrict__ grid) {
+  using C = typename cpx<R>::T;
+  extern __shared__ __align__(16) char smem[];
+  C* tw = (C*)smem;
+  C* buf = tw + a.ln.L;
+  C* res = buf + a.ln.L * (a.lpb + 1);
+  const int id = mix_id(a.total);
+  if (id < 0) return;
+  for (int i = threadIdx.x; i < a.ln.L; i += blockDim.x) tw[i] = ((const C*)a.tw)[i];
+  const Own o = own_of<true>(a);
+  const int c = (int)fdiv((uint32_t)id, a.dchunk), x = (id - c * a.nchunk) * a.lpb + o.l;
+  const bool xin = x < a.nx;
+  const size_t base = (size_t)(a.oall ? c : grid_pos(c, a.oN, a.oL, a.oNa)) * a.ost + (xin ? x : 0);
+  C* g = grid + base;
+  const C* lam = (const C*)a.lam + base;
+  const unsigned st = (unsigned)a.st;
+  mix_lines<R, false, true>(
+      a, o, buf, tw,
+      [&](int i, bool ok) {
+        C v{0, 0};
+        if (ok && xin && image_idx(i, a.N, a.ln.L, a.Na) >= 0) v = g[(unsigned)i * st];
+        return v;
+      },
+      [&](int i, C v) {
+        C f{0, 0};
+        if (xin) f = lam[(unsigned)i * st];
+        res[lds_at<true>(a, o.l, i)] = C{v.x * f.x - v.y * f.y, v.x * f.y + v.y * f.x};
+      });
+  __syncthreads();
+  mix_lines<R, true, true>(
+      a, o, buf, tw, [&](int i, bool) { return res[lds_at<true>(a, o.l, i)]; },
+      [&](int i, C v) {
+        if (xin && image_idx(i, a.N, a.ln.L, a.Na) >= 0) g[(unsigned)i * st] = v;
+      });
+}
+
 inline int mix_threads(const MixArgs& a) { return (a.lpb * a.ln.tpl + 63) / 64 * 64; }
 
 template <typename R>
@@ -541,6 +583,26 @@ size_t mix_lds_bytes(bool dbl, bool col, const MixLine& ln, int lpb) {
   const size_t L = (size_t)ln.L;
   const size_t n = L + (col ? L * (lpb + 1) : (size_t)lpb * (L + (L >> 4) + 1));
   return n * (dbl ? 16 : 8);
+}
+
+size_t mix_mul_lds_bytes(bool dbl, const MixLine& ln, int lpb) {
+  return mix_lds_bytes(dbl, true, ln, lpb) + (size_t)ln.L * (lpb + 1) * (dbl ? 16 : 8);
+}
+
+template <typename R>
+static hipError_t mul_go(const MixArgs& a, hipStream_t s, void* grid) {
+  const size_t lds = mix_mul_lds_bytes(sizeof(R) == 8, a.ln, a.lpb);
+  auto k = k_mix_mul<R>;
+  if (lds > 65536 &&
+      hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+    return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL(k, dim3((unsigned)(8 * ((a.total + 7) / 8))), dim3((unsigned)mix_threads(a)), lds, s, a,
+                     (typename cpx<R>::T*)grid);
+  return hipGetLastError();
+}
+
+hipError_t launch_mix_mul(bool dbl, const MixArgs& a, hipStream_t s, void* grid) {
+  return dbl ? mul_go<double>(a, s, grid) : mul_go<float>(a, s, grid);
 }
 
 hipError_t launch_mix_x(bool dbl, bool fwd, const MixArgs& a, hipStream_t s, const void* in, void* out) {

@@ -432,27 +432,34 @@ void k_spread3(KArgs a, const typename cpx<R>::T* __restrict__ fhat) {
   C* out = (C*)a.scratch + (size_t)item * G::SLOT;
   if (a.blocked3) {
     using B = Blocks3<W, G::T, G::TZ>;
-    // the right halo follows the tile's own cells (fewer than T in the last
-    // tile of a dimension that is not a multiple of it)
-    constexpr int m1 = W / 2 - 1;
-    const int hx = m1 + min(G::T, a.Nt[0] - it.x % a.ntiles[0] * G::T);
-    const int hy = m1 + min(G::T, a.Nt[1] - it.x / a.ntiles[0] % a.ntiles[1] * G::T);
-    const int hz = m1 + min(G::TZ, a.Nt[2] - it.x / a.ntiles[0] / a.ntiles[1] * G::TZ);
-    static_for<0, 27>([&](auto bc) {
-      constexpr int b = decltype(bc)::value;
-      constexpr int ex = B::ext(b % 3), ey = B::ext((b / 3) % 3), ez = B::ext(b / 9, G::TZ);
-      const int ox = b % 3 == 2 ? hx : B::org(b % 3), oy = (b / 3) % 3 == 2 ? hy : B::org((b / 3) % 3);
-      const int oz = b / 9 == 2 ? hz : B::org(b / 9, G::TZ);
-      constexpr int off = B::off(b), n = ex * ey * ez;
-      C* dst = out + off;
-      if constexpr (n > 0) {
-        for (int i = threadIdx.x; i < n; i += NT) {
-          const int lx = i % ex, q = i / ex;
-          const int lz = q % ez, ly = q / ez;
-          dst[i] = SpreadCell<R>::get(tile, G::CELLS, (ox + lx) + G::SX * (oy + ly) + G::SXY * (oz + lz), inv);
+    auto flush = [&](auto rag, int hx, int hy, int hz) {
+      static_for<0, 27>([&](auto bc) {
+        constexpr int b = decltype(bc)::value;
+        constexpr int ex = B::ext(b % 3), ey = B::ext((b / 3) % 3), ez = B::ext(b / 9, G::TZ);
+        constexpr bool R3 = decltype(rag)::value;
+        const int ox = R3 && b % 3 == 2 ? hx : B::org(b % 3), oy = R3 && (b / 3) % 3 == 2 ? hy : B::org((b / 3) % 3);
+        const int oz = R3 && b / 9 == 2 ? hz : B::org(b / 9, G::TZ);
+        constexpr int off = B::off(b), n = ex * ey * ez;
+        C* dst = out + off;
+        if constexpr (n > 0) {
+          for (int i = threadIdx.x; i < n; i += NT) {
+            const int lx = i % ex, q = i / ex;
+            const int lz = q % ez, ly = q / ez;
+            dst[i] = SpreadCell<R>::get(tile, G::CELLS, (ox + lx) + G::SX * (oy + ly) + G::SXY * (oz + lz), inv);
+          }
         }
-      }
-    });
+      });
+    };
+    if (a.blocked3 == 1) {  // whole tiles: constant origins
+      flush(std::false_type{}, 0, 0, 0);
+    } else {
+      // the right halo follows the tile's own cells (fewer than T in the last
+      // tile of a dimension that is not a multiple of it)
+      constexpr int m1 = W / 2 - 1;
+      flush(std::true_type{}, m1 + min(G::T, a.Nt[0] - it.x % a.ntiles[0] * G::T),
+            m1 + min(G::T, a.Nt[1] - it.x / a.ntiles[0] % a.ntiles[1] * G::T),
+            m1 + min(G::TZ, a.Nt[2] - it.x / a.ntiles[0] / a.ntiles[1] * G::TZ));
+    }
     return;
   }
   const int px = threadIdx.x & 31;

@@ -110,8 +110,9 @@ struct KArgs {
   int nitems;
   const char* rec;    // node records in sorted order (NodeRec layout), tiled plans
   int recBytes;
-  int blocked3;       // 3-D scratch slots stored as 27 halo/interior blocks; 2-D: every grid
-                      // point is covered by its own tile and neighbouring ones only (k_fold2)
+  int blocked3;       // 3-D scratch slots stored as 27 halo/interior blocks (1: whole tiles, 2: some
+                      // partial); 2-D: every grid point is covered by its own tile and neighbouring
+                      // ones only (k_fold2)
   int tvar;           // 3-D tile geometry variant (compile-time tile edge)
   int fix2;           // FP32 2-D spreading accumulates packed fixed point (one
                       // 64-bit LDS atomic per tap) instead of two FP64 planes

@@ -58,6 +58,7 @@ struct MixArgs {
   // s % Bsl + (s / Bsl) Bsl P, its grid is slot nsl - 1 - (s - s0)
   int s0, nsl;
   long long Bsl, P, Q;
+  const void* lam;  // launch_mix_mul: the grid-sized factor
 };
 
 // Radices of a line of L points; false where the passes are not built for it
@@ -69,5 +70,9 @@ int mix_shape(bool dbl, bool col, const MixLine& ln, long long lines, long long 
 size_t mix_lds_bytes(bool dbl, bool col, const MixLine& ln, int lpb);
 hipError_t launch_mix_x(bool dbl, bool fwd, const MixArgs& a, hipStream_t s, const void* in, void* out);
 hipError_t launch_mix_col(bool dbl, bool fwd, const MixArgs& a, hipStream_t s, void* grid);
+// Strided pass along the last dimension in place: forward FFT of the image
+// positions, product with lam, inverse FFT, image positions written.
+size_t mix_mul_lds_bytes(bool dbl, const MixLine& ln, int lpb);
+hipError_t launch_mix_mul(bool dbl, const MixArgs& a, hipStream_t s, void* grid);
 
 }  // namespace nfftm

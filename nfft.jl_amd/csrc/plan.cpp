@@ -407,6 +407,81 @@ struct DevBuf {
 
 }  // namespace
 
+// Pass over the lines of dimension d of a D-dimensional grid of L points (images
+// of N at the positions that na gives), nsl of them per launch.
+static MixArgs mix_pass_args(bool dbl, int D, const i64* N, const i64* L, const i64* na, const double* const* fac,
+                             const MixLine& ln, const void* tw, int d, int nsl) {
+  MixArgs a;
+  std::memset(&a, 0, sizeof a);
+  i64 n[3] = {1, 1, 1}, l[3] = {1, 1, 1}, gs[4] = {1, 1, 1, 1};
+  a.P = a.Q = 1;
+  for (int e = 0; e < 3; ++e) {
+    if (e < D) {
+      n[e] = N[e];
+      l[e] = L[e];
+      a.fac[e] = fac[e];
+    }
+    gs[e + 1] = gs[e] * l[e];
+    a.P *= n[e];
+    a.Q *= l[e];
+  }
+  a.ln = ln;
+  a.tw = tw;
+  a.N = (int)n[d];
+  a.Na = (int)na[d];
+  a.st = gs[d];
+  if (d == 0) {
+    a.nlines = (int)(n[1] * n[2]);
+    a.lpb = mix_shape(dbl, false, a.ln, a.nlines, nsl);
+    a.total = (a.nlines + a.lpb - 1) / a.lpb;
+  } else {
+    const int o = 3 - d;
+    a.oall = d == 2;
+    a.oN = (int)n[o];
+    a.oL = (int)l[o];
+    a.oNa = (int)na[o];
+    a.ost = gs[o];
+    a.nx = (int)l[0];
+    const i64 outer = a.oall ? l[o] : n[o];
+    a.lpb = mix_shape(dbl, true, a.ln, a.nx, outer * nsl);
+    a.nchunk = (a.nx + a.lpb - 1) / a.lpb;
+    a.total = (int)(a.nchunk * outer);
+  }
+  while ((1 << a.lsh) < a.lpb) ++a.lsh;
+  a.dchunk = make_fastdiv((uint32_t)std::max(1, a.nchunk));
+  a.dN1 = make_fastdiv((uint32_t)n[1]);
+  a.N1 = (int)n[1];
+  a.L1 = (int)l[1];
+  a.Na1 = (int)na[1];
+  a.st1 = gs[1];
+  a.N2 = (int)n[2];
+  a.L2 = (int)l[2];
+  a.Na2 = (int)na[2];
+  a.st2 = gs[2];
+  a.oscale = 1.0;
+  a.ist = 1;
+  a.nsl = 1;
+  a.Bsl = 1;
+  return a;
+}
+
+// Appends the (cos, sin)(2 pi k / L), k < L, of the precision to a host table.
+static void append_twiddles(std::vector<char>& h, i64 L, bool dbl) {
+  const size_t o = h.size(), es = dbl ? 16 : 8;
+  h.resize(o + (size_t)L * es);
+  for (i64 k = 0; k < L; ++k) {
+    const double th = 2.0 * M_PI * (double)k / (double)L, c = std::cos(th), sn = std::sin(th);
+    char* e = h.data() + o + (size_t)k * es;
+    if (dbl) {
+      ((double*)e)[0] = c;
+      ((double*)e)[1] = sn;
+    } else {
+      ((float*)e)[0] = (float)c;
+      ((float*)e)[1] = (float)sn;
+    }
+  }
+}
+
 // ===========================================================================
 // The plan
 // ===========================================================================
@@ -637,6 +712,8 @@ struct nfftm_plan_s {
     a.nitems = nitems;
     a.rec = d_rec.p;
     a.blocked3 = blocked3() ? 1 : 0;
+    for (int d = 0; d < D && a.blocked3 && D == 3; ++d)
+      if (Nt[d] % T[d]) a.blocked3 = 2;
     a.tvar = tvar;
     // FP32 2-D spreading in packed fixed point where the deconvolution does
     // not amplify its rounding much (sigma near 2 or above; at small sigma the
@@ -684,59 +761,19 @@ struct nfftm_plan_s {
 
   // Pass over the lines of dimension d (k_mixfft.hip).
   MixArgs mixargs(int d) const {
-    MixArgs a;
-    std::memset(&a, 0, sizeof a);
-    i64 n[3] = {1, 1, 1}, l[3] = {1, 1, 1}, na[3] = {0, 0, 0}, gs[4] = {1, 1, 1, 1}, off = 0;
-    for (int e = 0; e < 3; ++e) {
-      if (e < D) {
-        n[e] = N[e];
-        l[e] = Nt[e];
-        na[e] = N[e] / 2;
-        a.fac[e] = d_deconv.p + off;
-        off += N[e];
-      }
-      gs[e + 1] = gs[e] * l[e];
+    i64 na[3] = {0, 0, 0};
+    const double* fac[3] = {nullptr, nullptr, nullptr};
+    i64 off = 0;
+    for (int e = 0; e < D && e < 3; ++e) {
+      na[e] = N[e] / 2;
+      fac[e] = d_deconv.p + off;
+      off += N[e];
     }
-    a.ln = mixln[d];
-    a.tw = d_tw.p + tw_off[d];
-    a.N = (int)n[d];
-    a.Na = (int)na[d];
-    a.st = gs[d];
-    if (d == 0) {
-      a.nlines = (int)(n[1] * n[2]);
-      a.lpb = mix_shape(dbl(), false, a.ln, a.nlines, sln);
-      a.total = (a.nlines + a.lpb - 1) / a.lpb;
-    } else {
-      const int o = 3 - d;
-      a.oall = d == 2;
-      a.oN = (int)n[o];
-      a.oL = (int)l[o];
-      a.oNa = (int)na[o];
-      a.ost = gs[o];
-      a.nx = (int)l[0];
-      const i64 outer = a.oall ? l[o] : n[o];
-      a.lpb = mix_shape(dbl(), true, a.ln, a.nx, outer * sln);
-      a.nchunk = (a.nx + a.lpb - 1) / a.lpb;
-      a.total = (int)(a.nchunk * outer);
-    }
-    while ((1 << a.lsh) < a.lpb) ++a.lsh;
-    a.dchunk = make_fastdiv((uint32_t)std::max(1, a.nchunk));
-    a.dN1 = make_fastdiv((uint32_t)n[1]);
-    a.N1 = (int)n[1];
-    a.L1 = (int)l[1];
-    a.Na1 = (int)na[1];
-    a.st1 = gs[1];
-    a.N2 = (int)n[2];
-    a.L2 = (int)l[2];
-    a.Na2 = (int)na[2];
-    a.st2 = gs[2];
-    a.oscale = 1.0;
+    MixArgs a = mix_pass_args(dbl(), D, N, Nt, na, fac, mixln[d], d_tw.p + tw_off[d], d, sln);
     a.ist = io_stride;
     a.s0 = sl0;
     a.nsl = sln;
     a.Bsl = io_stride;
-    a.P = P;
-    a.Q = Q;
     return a;
   }
 
@@ -1031,7 +1068,12 @@ int set_nodes(nfftm_plan_s& p, const double* k, bool rows, i64 M, bool keep) {
   while (((i64)1 << a.key_bits) < ntile) ++a.key_bits;
   int nitems = 0, nmulti = 0;
   HIPCHK(w.stats.ensure(4));
-  if (!w.h_stats) HIPCHK(hipHostMalloc((void**)&w.h_stats, 4 * sizeof(int), hipHostMallocDefault));
+  // pinned where nodes! comes again (its allocation costs a plan more than it saves once)
+  int hs[4] = {0, 0, 0, 0}, *hp = hs;
+  if (keep) {
+    if (!w.h_stats) HIPCHK(hipHostMalloc((void**)&w.h_stats, 4 * sizeof(int), hipHostMallocDefault));
+    hp = w.h_stats;
+  }
   if (!p.tiled) {
     HIPCHK(launch_check_nodes(kd, (i64)D * M, w.stats.p + 3, st));
   } else {
@@ -1044,12 +1086,12 @@ int set_nodes(nfftm_plan_s& p, const double* k, bool rows, i64 M, bool keep) {
     HIPCHK(launch_bin_keys(a, k0, w.key_in.p, w.idx_in.p, w.cnt.p, st));
     HIPCHK(launch_bin_scan(a, w.cnt.p, w.off.p, w.ioff.p, w.stats.p, st));
   }
-  HIPCHK(hipMemcpyAsync(w.h_stats, w.stats.p, 4 * sizeof(int), hipMemcpyDeviceToHost, st));
+  HIPCHK(hipMemcpyAsync(hp, w.stats.p, 4 * sizeof(int), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
-  if (w.h_stats[3]) return bad_node();
+  if (hp[3]) return bad_node();
   if (p.tiled) {
-    nitems = w.h_stats[0];
-    nmulti = w.h_stats[1];
+    nitems = hp[0];
+    nmulti = hp[1];
   }
   // from here on the plan has the new nodes
   p.M = M;
@@ -1483,30 +1525,13 @@ int create_impl(nfftm_plan_s& p, const double* k) {
   if (p.pfft || p.mix) {
     // twiddle tables exp(-2 pi i k / Nt_d) as (cos, sin) of 2 pi k / Nt_d,
     // FP64 on the host, stored in the data precision
-    const size_t es = p.dbl() ? 16 : 8;
-    size_t bytes = 0;
+    std::vector<char> h;
     for (int d = 0; d < p.D; ++d) {
-      p.tw_off[d] = bytes;
-      bytes += (size_t)p.Nt[d] * es;
+      p.tw_off[d] = h.size();
+      append_twiddles(h, p.Nt[d], p.dbl());
     }
-    std::vector<char> h(bytes);
-    for (int d = 0; d < p.D; ++d) {
-      const i64 L = p.Nt[d];
-      for (i64 k = 0; k < L; ++k) {
-        const double th = 2.0 * M_PI * (double)k / (double)L;
-        const double c = std::cos(th), sn = std::sin(th);
-        char* e = h.data() + p.tw_off[d] + (size_t)k * es;
-        if (p.dbl()) {
-          ((double*)e)[0] = c;
-          ((double*)e)[1] = sn;
-        } else {
-          ((float*)e)[0] = (float)c;
-          ((float*)e)[1] = (float)sn;
-        }
-      }
-    }
-    HIPCHK(p.d_tw.alloc(bytes));
-    HIPCHK(hipMemcpy(p.d_tw.p, h.data(), bytes, hipMemcpyHostToDevice));
+    HIPCHK(p.d_tw.alloc(h.size()));
+    HIPCHK(hipMemcpy(p.d_tw.p, h.data(), h.size(), hipMemcpyHostToDevice));
   }
   if (p.f1) {
     // (cos, sin)(2 pi j / n1) and (2 pi j / Lm) in the data precision,
@@ -2661,7 +2686,19 @@ struct nfftm_toeplitz_s {
   hipStream_t stream = nullptr;
   std::unique_ptr<FFTStage> fft;
   DevBuf<char> x;
+  // products on line passes (D >= 2, sizes they are built for): radices,
+  // twiddles, and the factors 1 of the dimension-1 passes
+  bool mix = false;
+  MixLine ln[3];
+  DevBuf<char> tw;
+  size_t tw_off[3] = {0, 0, 0};
+  DevBuf<double> one;
   bool dbl() const { return prec == NFFTM_F64; }
+  MixArgs margs(int d) const {
+    const i64 na[3] = {0, 0, 0};
+    const double* fac[3] = {one.p, nullptr, nullptr};
+    return mix_pass_args(dbl(), D, N, L, na, fac, ln[d], tw.p + tw_off[d], d, 1);
+  }
   size_t celem() const { return dbl() ? 16 : 8; }
   ToepArgs targs() const {
     ToepArgs a;
@@ -2699,6 +2736,22 @@ int nfftm_toeplitz_create(nfftm_toeplitz* out, int prec, int D, const int64_t* N
   HIPCHK(t->x.alloc((size_t)t->Q * t->celem()));
   t->fft.reset(new FFTStage());
   if (int rc = t->fft->build(D, t->L, t->dbl())) return rc;
+  t->mix = D >= 2 && t->Q < (1LL << 31);
+  for (int d = 0; d < D && t->mix; ++d) t->mix = mix_factor(t->L[d], t->dbl(), false, &t->ln[d]);
+  if (t->mix) {
+    std::vector<char> h;
+    for (int d = 0; d < D; ++d) {
+      t->tw_off[d] = h.size();
+      append_twiddles(h, t->L[d], t->dbl());
+    }
+    HIPCHK(t->tw.alloc(h.size()));
+    HIPCHK(hipMemcpy(t->tw.p, h.data(), h.size(), hipMemcpyHostToDevice));
+    const std::vector<double> ones((size_t)t->N[0], 1.0);
+    HIPCHK(t->one.alloc(ones.size()));
+    HIPCHK(hipMemcpy(t->one.p, ones.data(), ones.size() * sizeof(double), hipMemcpyHostToDevice));
+    const MixArgs a = t->margs(D - 1);
+    t->mix = mix_mul_lds_bytes(t->dbl(), a.ln, a.lpb) <= 163840;
+  }
   *out = t.release();
   return NFFTM_OK;
 }
@@ -2730,6 +2783,21 @@ int nfftm_toeplitz_apply(nfftm_toeplitz t, const void* lambda, void* y) {
   const bool dbl = t->dbl();
   const ToepArgs a = t->targs();
   hipStream_t s = t->stream;
+  if (t->mix) {
+    // 2 D - 1 pruned line passes: the padding and cropping in the dimension-1
+    // passes, the product in the last dimension's (separate kernels around
+    // rocFFT: 7 launches in 2-D and three more passes over the grid)
+    MixArgs x = t->margs(0);
+    HIPCHK(launch_mix_x(dbl, true, x, s, y, t->x.p));
+    for (int d = 1; d < t->D - 1; ++d) HIPCHK(launch_mix_col(dbl, true, t->margs(d), s, t->x.p));
+    MixArgs m = t->margs(t->D - 1);
+    m.lam = lambda;
+    HIPCHK(launch_mix_mul(dbl, m, s, t->x.p));
+    for (int d = t->D - 2; d >= 1; --d) HIPCHK(launch_mix_col(dbl, false, t->margs(d), s, t->x.p));
+    x.oscale = 1.0 / (double)t->Q;
+    HIPCHK(launch_mix_x(dbl, false, x, s, t->x.p, y));
+    return NFFTM_OK;
+  }
   HIPCHK(launch_pad_corner(dbl, y, t->x.p, a, s));
   if (int rc = t->fft->exec(true, t->x.p, t->celem(), s)) return rc;
   HIPCHK(launch_cmul(dbl, t->x.p, lambda, t->Q, s));
