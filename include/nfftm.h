@@ -156,7 +156,8 @@ int nfftm_adjoint(nfftm_plan p, const void* fhat_dev, void* f_dev);
  * pullback of y = A(k) f is then (kbar, adjoint(p) * ybar).  Computed as the
  * forward path (deconvolve!, forward FFT) followed by a gather with the
  * analytic derivative of the Kaiser-Bessel window (of the fitted polynomial
- * in POLYNOMIAL/TENSOR mode), window arithmetic in FP64.
+ * in POLYNOMIAL/TENSOR mode), window arithmetic in FP64.  An FP32 plan's
+ * gradient is gathered from its FP32 grid and carries FP32 digits, in FP64.
  * f: prod(N) complex, ybar: M complex, kbar: D*M doubles laid out as k
  * (column-major D x M, caller's node order); all device pointers.  Uses the
  * plan's grid. */

@@ -569,6 +569,11 @@ struct nfftm_plan_s {
   // the same passes with per-plan radices (other grids): line radices
   bool mix = false;
   MixLine mixln[3];
+  // Forward transforms take them in FP64, and in FP32 on directional plans.
+  // An ordinary FP32 plan's forward grid also gives the node gradient, whose
+  // result is FP64: there the passes move it by FP32 rounding (2e-7), so its
+  // forward FFT stays rocFFT's.
+  bool mix_forward() const { return mix && (dbl() || dir()); }
   DevBuf<char> d_tw;
   size_t tw_off[3] = {0, 0, 0};
   // 1-D grids of n1 Lm^2 points: the three-pass FFT of k_fft1.hip, its
@@ -1379,7 +1384,7 @@ int forward_to_grid(nfftm_plan_s& p, const void* f, Mark&& mark) {
     HIPCHK(launch_pruned_fft_fwd(p.dbl(), a, p.stream, f, p.d_grid.p, 1));
     return NFFTM_OK;
   }
-  if (p.mix) {
+  if (p.mix_forward()) {
     {
       ProfScope ps(p, 0);
       HIPCHK(launch_mix_x(p.dbl(), true, p.mixargs(0), p.stream, f, p.d_grid.p));

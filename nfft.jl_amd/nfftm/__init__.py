@@ -441,7 +441,8 @@ class NFFTPlan:
         """Node gradient kbar[d, j] = Re(conj(ybar_j) * d fHat_j / d k[d, j]) of
         fHat = p * f: the node cotangent that the reference's rrule leaves as
         NoTangent() (AbstractNFFTs/ext/AbstractNFFTsChainRulesCoreExt.jl:14-45).
-        Returns a (D, M) float64 device tensor in the axis order of k."""
+        Returns a (D, M) float64 device tensor in the axis order of k; an FP32
+        plan gathers it from its FP32 grid, so its digits are FP32's."""
         if self.directional:  # as the library answers (NFFTM_ERR_UNSUPPORTED)
             raise NFFTError("node gradient of a directional plan")
         f = self._prep(f, self.N, "f")
