@@ -25,7 +25,7 @@ struct Geo3 {
     return ((2 * (size_t)sx_of(t) * pad_of(t) * pad_of(tz) * sizeof(R)) + 15) & ~(size_t)15;
   }
   static constexpr __host__ __device__ size_t batch_bytes(int nb) { return (size_t)nb * RB + (size_t)nb * 2 * sizeof(R); }
-  static constexpr size_t CAP = V == 0 ? 163840 : 81920;
+  static constexpr size_t CAP = V != 1 ? 163840 : 81920;
   // V = 1 choice, encoded t * 32 + tz
   static constexpr __host__ __device__ int flat_tile() {
     int best = 4 * 32 + 4, vol = 0;
@@ -43,9 +43,11 @@ struct Geo3 {
   static constexpr int TC = sizeof(R) == 4 ? (W <= 10 ? 16 : W <= 12 ? 12 : W <= 14 ? 10 : 8)
                                            : (W <= 8 ? 12 : W <= 12 ? 8 : W <= 14 ? 6 : 4);
   // FP64, W = 10: twice as long along z (halo 7.1 instead of 9.6 slots per
-  // grid, still with a batch of records in the LDS of the interpolation)
-  static constexpr int T = V == 0 ? TC : flat_tile() / 32;
-  static constexpr int TZ = V == 0 ? (sizeof(R) == 8 && W == 10 ? 16 : TC) : flat_tile() % 32;
+  // grid, still with a batch of records in the LDS of the interpolation);
+  // V = 2 is the cubic tile of this width (short_tile3 in plan.cpp)
+  static constexpr bool LONG = sizeof(R) == 8 && W == 10;
+  static constexpr int T = V != 1 ? TC : flat_tile() / 32;
+  static constexpr int TZ = V == 0 ? (LONG ? 16 : TC) : V == 2 ? TC : flat_tile() % 32;
   static constexpr int P = T + W - 1;
   static constexpr int PZ = TZ + W - 1;
   static constexpr int SX = sx_of(T);  // W = 8: 8x8 lanes on distinct banks
@@ -61,7 +63,7 @@ struct Geo3 {
   static constexpr size_t FV_OFF = (size_t)NB * RB;
   static constexpr size_t TILE_OFF = FV_OFF + (size_t)NB * 2 * sizeof(R);
   static constexpr size_t LDS = TILE_OFF + TILE_BYTES;
-  static constexpr bool VALID = LDS <= CAP;
+  static constexpr bool VALID = LDS <= CAP && (V != 2 || LONG);
   static_assert(TILE_OFF % 16 == 0, "tile offset");
 
 };
@@ -973,6 +975,7 @@ static hipError_t fold_fft3_l(const KArgs& a, const FArgs& f, hipStream_t s, voi
 
 template <typename R, int W>
 static hipError_t fold_fft3_v(const KArgs& a, const FArgs& f, hipStream_t s, void* grid, bool dry) {
+  if (a.tvar == 2) return hipErrorNotSupported;  // lines of at least 128 points hold the long tile
   return a.tvar ? fold_fft3_l<R, W, 1>(a, f, s, grid, dry) : fold_fft3_l<R, W, 0>(a, f, s, grid, dry);
 }
 
@@ -1031,7 +1034,11 @@ static hipError_t go3(bool spread, int NT, const KArgs& a, hipStream_t s, const 
 
 template <typename R, int W>
 static hipError_t go3v(bool spread, int NT, const KArgs& a, hipStream_t s, const void* in, void* out) {
-  return a.tvar ? go3<R, W, 1>(spread, NT, a, s, in, out) : go3<R, W, 0>(spread, NT, a, s, in, out);
+  switch (a.tvar) {
+    case 0: return go3<R, W, 0>(spread, NT, a, s, in, out);
+    case 1: return go3<R, W, 1>(spread, NT, a, s, in, out);
+    default: return go3<R, W, 2>(spread, NT, a, s, in, out);
+  }
 }
 
 template <typename R>
@@ -1074,6 +1081,7 @@ static hipError_t fold3(const KArgs& a, hipStream_t s, void* grid) {
 hipError_t launch_fold_d3(bool dbl, int W, const KArgs& a, hipStream_t s, void* grid) {
 #define NFFTM_F3(WW)                                                                          \
   case WW:                                                                                    \
+    if (a.tvar == 2) return dbl ? fold3<double, WW, 2>(a, s, grid) : fold3<float, WW, 2>(a, s, grid); \
     if (a.tvar) return dbl ? fold3<double, WW, 1>(a, s, grid) : fold3<float, WW, 1>(a, s, grid); \
     return dbl ? fold3<double, WW, 0>(a, s, grid) : fold3<float, WW, 0>(a, s, grid);
   switch (W) {
@@ -1117,10 +1125,12 @@ static void geo3(int W, int* T, size_t* lds, int* P, int* SX, bool* valid) {
 
 void tile3_geometry(bool dbl, int W, int V, int* T, size_t* lds, int* P, int* SX, bool* valid) {
   if (dbl) {
-    if (V) geo3<double, 1>(W, T, lds, P, SX, valid);
+    if (V == 2) geo3<double, 2>(W, T, lds, P, SX, valid);
+    else if (V) geo3<double, 1>(W, T, lds, P, SX, valid);
     else geo3<double, 0>(W, T, lds, P, SX, valid);
   } else {
-    if (V) geo3<float, 1>(W, T, lds, P, SX, valid);
+    if (V == 2) geo3<float, 2>(W, T, lds, P, SX, valid);
+    else if (V) geo3<float, 1>(W, T, lds, P, SX, valid);
     else geo3<float, 0>(W, T, lds, P, SX, valid);
   }
 }

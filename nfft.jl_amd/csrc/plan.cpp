@@ -887,6 +887,20 @@ bool set_tile_shape(nfftm_plan_s& p, int t) {
 // path.
 bool tiles_ok(const nfftm_plan_s& p);
 
+// Whether variant 0 of a width with a long tile (FP64, 2m = 10: 8 x 8 x 16)
+// takes the cubic one (8^3): where the grid does not hold the long tile's
+// padded edge (it would be left to the node-parallel kernels: 9 .. 12 slices
+// of 96^2, 2 10^5 nodes: adjoint 18.3 ms instead of 0.2), and below 1024 long
+// tiles, which leave most of the chip idle (sigma = 2, us of interpolation +
+// spreading with the fold, cubic / long: 24^3 image, 200 nodes 34 / 52, 5 10^4
+// nodes 77 / 149; 48^3, 864 long tiles, 36 / 55, 124 / 127; 64^3, 2048 of
+// them, 36 / 46, 277 / 199).
+bool short_tile3(const nfftm_plan_s& p, const int* T, const int* P) {
+  i64 n = 1;
+  for (int d = 0; d < 3; ++d) n *= (p.Nt[d] + T[d == 2] - 1) / T[d == 2];
+  return p.Nt[2] < P[1] || n < 1024;
+}
+
 // 3-D geometry of variant V (compile-time tile of k_tile3.hip); false if
 // that variant has no tile fitting its LDS budget.
 bool set_tile3(nfftm_plan_s& p, int V) {
@@ -894,6 +908,10 @@ bool set_tile3(nfftm_plan_s& p, int V) {
   size_t lds = 0;
   bool valid = false;
   tile3_geometry(p.dbl(), p.W, V, T, &lds, P, &SX, &valid);
+  if (V == 0 && valid && T[1] > T[0] && short_tile3(p, T, P)) {
+    V = 2;
+    tile3_geometry(p.dbl(), p.W, V, T, &lds, P, &SX, &valid);
+  }
   if (!valid) return false;
   p.tvar = V;
   for (int d = 0; d < 3; ++d) {
