@@ -505,7 +505,7 @@ struct nfftm_plan_s {
   // plan's own work vectors are contiguous)
   i64 io_stride = 1;
   // slices of the running launches (1 outside a directional transform), and
-  // how many of them d_grid and d_scratch hold
+  // how many of them d_grid and d_scratch (d_fsort) hold
   int sl0 = 0, sln = 1, gcap = 1, scap = 1;
   // 3-D scratch slots in halo/interior block layout: halos (m - 1, m cells)
   // no wider than any tile, a partial last one included
@@ -1006,25 +1006,60 @@ int build_records(nfftm_plan_s& p) {
 }
 
 // Directional plans on the 1-D and 2-D tile kernels run several slices per
-// launch: as many grids as fit 512 MiB and as many scratch areas as fit
-// another 512 MiB, at most 256 of each (one slice of a 480^2 grid takes about
-// 9 us of launches and latency per kernel, eight kernels; 32 of them together
-// fill the GPU).  The 3-D kernels and the three-pass 1-D FFT fill it with one.
+// launch: as many grids as fit 512 MiB, and as many scratch areas and sorted
+// node values as fit 512 MiB each, at most 256 (one slice of a 480^2 grid takes
+// about 9 us of launches and latency per kernel, eight kernels; 32 of them
+// together fill the GPU), fewer where the device has not that much memory.
+// The 3-D kernels and the three-pass 1-D FFT fill it with one.
 constexpr size_t SLICE_BYTES = (size_t)512 << 20;
 int slice_cap(const nfftm_plan_s& p, size_t bytes) {
   if (!p.dir() || !p.tiled || p.D == 3 || p.f1 || p.Bsl > 0x7fffffff || p.Asl > 0x7fffffff / p.Bsl) return 1;
   return (int)std::max<i64>(1, std::min<i64>({p.Bsl * p.Asl, 256, (i64)(SLICE_BYTES / std::max<size_t>(1, bytes))}));
 }
-int alloc_grid(nfftm_plan_s& p) {
-  p.gcap = slice_cap(p, (size_t)p.Q * p.celem());
-  HIPCHK(p.d_grid.alloc((size_t)p.gcap * p.Q * p.celem()));
-  return NFFTM_OK;
+// fn(n), which allocates for n slices: n = cap, or half as many as long as the
+// memory does not suffice.
+template <typename F>
+int alloc_slices(int cap, int* got, F&& fn) {
+  for (;; cap = (cap + 1) / 2) {
+    const hipError_t e = fn(cap);
+    if (e == hipErrorOutOfMemory && cap > 1) {
+      (void)hipGetLastError();
+      continue;
+    }
+    HIPCHK(e);
+    *got = cap;
+    return NFFTM_OK;
+  }
 }
+int alloc_grid(nfftm_plan_s& p, int most = 256) {
+  const size_t one = (size_t)p.Q * p.celem();
+  return alloc_slices(std::min(most, slice_cap(p, one)), &p.gcap, [&](int n) { return p.d_grid.alloc(n * one); });
+}
+// Scratch areas and (1-D polynomial windows) sorted values of the plan's nodes.
 int alloc_scratch(nfftm_plan_s& p) {
   const size_t one = std::max<size_t>(1, (size_t)p.nitems) * p.slot_cells() * p.celem();
-  p.scap = slice_cap(p, one);
-  HIPCHK(p.d_scratch.ensure((size_t)p.scap * one));
-  return NFFTM_OK;
+  const size_t srt = p.sorted_io() ? (size_t)p.M * p.celem() : 0;
+  return alloc_slices(slice_cap(p, std::max(one, srt)), &p.scap, [&](int n) {
+    hipError_t e = p.d_scratch.ensure(n * one);
+    if (e == hipSuccess && srt) e = p.d_fsort.ensure(n * srt);
+    if (e != hipSuccess) {
+      p.d_scratch.reset();
+      p.d_fsort.reset();
+    }
+    return e;
+  });
+}
+// The buffers of a plan that has just become directional.
+int grow_slices(nfftm_plan_s& p) {
+  if (int rc = alloc_grid(p)) return rc;
+  if (!p.tiled) return NFFTM_OK;
+  int rc = alloc_scratch(p);
+  if (rc == NFFTM_ERR_OOM && p.gcap > 1) {  // the grids have taken what the scratch needs
+    g_err.clear();
+    (void)hipGetLastError();
+    if ((rc = alloc_grid(p, 1)) == NFFTM_OK) rc = alloc_scratch(p);
+  }
+  return rc;
 }
 
 // sort, split each tile's nodes into work items, gather the shifted nodes in
@@ -1165,7 +1200,6 @@ int set_nodes(nfftm_plan_s& p, const double* k, bool rows, i64 M, bool keep) {
     if (p.sorted_io()) p.d_rec.reset();
     else if (int rc = build_records(p)) return rc;
     if (p.sorted_io() && M > 0) {
-      HIPCHK(p.d_fsort.ensure((size_t)p.scap * M * p.celem()));
       HIPCHK(p.d_iperm.ensure((size_t)M));
       HIPCHK(launch_inv_perm(p.d_perm.p, p.d_iperm.p, M, p.stream));
     }
@@ -2085,11 +2119,7 @@ int nfftm_plan_create_dims(nfftm_plan* out, int prec, int D, const int64_t* N, i
       if (d > dim_hi) p->Asl *= N[d];
     }
     std::unique_ptr<nfftm_plan_s> own(p);
-    if (int rc = alloc_grid(*p)) return rc;
-    if (p->tiled) {
-      if (int rc = alloc_scratch(*p)) return rc;
-      if (p->d_fsort.p) HIPCHK(p->d_fsort.alloc((size_t)p->scap * p->M * p->celem()));
-    }
+    if (int rc = grow_slices(*p)) return rc;
     own.release();
   }
   *out = p;
@@ -2459,14 +2489,17 @@ int nfftm_plan_copy(nfftm_plan src, nfftm_plan* dst) {
   p->M = src->M;
   p->stream = src->stream;
   for (int d = 0; d < src->D; ++d) p->N[d] = src->N[d];
-  p->Dfull = src->Dfull;
-  p->dlo = src->dlo;
-  p->Bsl = src->Bsl;
-  p->Asl = src->Asl;
-  for (int d = 0; d < MAXD; ++d) p->Nfull[d] = src->Nfull[d];
   std::vector<double> k;
   if (int rc = host_nodes(*src, &k)) return rc;
   if (int rc = create_impl(*p, k.data())) return rc;
+  if (src->dir()) {
+    p->Dfull = src->Dfull;
+    p->dlo = src->dlo;
+    p->Bsl = src->Bsl;
+    p->Asl = src->Asl;
+    for (int d = 0; d < MAXD; ++d) p->Nfull[d] = src->Nfull[d];
+    if (int rc = grow_slices(*p)) return rc;
+  }
   std::memcpy(p->timing, src->timing, sizeof p->timing);
   *dst = p.release();
   return NFFTM_OK;
