@@ -1080,9 +1080,15 @@ int set_nodes(nfftm_plan_s& p, const double* k, bool rows, i64 M, bool keep) {
     nfftm_plan_s& p;
     bool keep;
     ~Release() {
-      if (!keep) p.bw.release();
+      if (keep) return;
+      (void)hipStreamSynchronize(p.stream);  // the kernels that use them
+      p.bw.release();
     }
   } release{p, keep};
+  // The node arrays are rewritten in place, and the plan's own stream is not
+  // the only one that reads them: a batch holds their addresses and runs on its
+  // caller's.  (gen = 0: a plan under construction, nothing reads it yet.)
+  if (p.gen > 0) HIPCHK(hipDeviceSynchronize());
   if (k) {
     HIPCHK(w.k.ensure((size_t)D * M));
     if (M) HIPCHK(hipMemcpyAsync(w.k.p, k, (size_t)D * M * sizeof(double), hipMemcpyHostToDevice, st));
@@ -2130,7 +2136,6 @@ int nfftm_nodes(nfftm_plan p, const double* k_host, int64_t M) {
   g_err.clear();
   if (!p) return fail(NFFTM_ERR_ARG, "plan is NULL");
   if (M > 0 && !k_host) return fail(NFFTM_ERR_ARG, "k is NULL");
-  HIPCHK(hipStreamSynchronize(p->stream));
   return set_nodes(*p, k_host, false, M, true);
 }
 
@@ -2138,7 +2143,6 @@ int nfftm_nodes_rows(nfftm_plan p, const double* k_host, int64_t M) {
   g_err.clear();
   if (!p) return fail(NFFTM_ERR_ARG, "plan is NULL");
   if (M > 0 && !k_host) return fail(NFFTM_ERR_ARG, "k is NULL");
-  HIPCHK(hipStreamSynchronize(p->stream));
   return set_nodes(*p, k_host, true, M, true);
 }
 
