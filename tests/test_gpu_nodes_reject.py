@@ -1,7 +1,8 @@
 """nodes! with a node outside [-1/2, 1/2] or NaN (checkNodes, src/utils.jl:46-55),
-which the binning kernels find on the device: ArgumentError, and the plan goes
-on with its old nodes (forward bit for bit, adjoint FP32 rel-l2 <= 1e-6); a
-following nodes! with valid nodes and another M equals a fresh plan.
+found by the binning kernels on the device (by a kernel of its own, or on the
+host, for node-parallel plans): ArgumentError, and the plan goes on with its old
+nodes (forward bit for bit, adjoint FP32 rel-l2 <= 1e-6); a following nodes!
+with valid nodes and another M equals a fresh plan.
 
 Both layouts of the entry point (rows, as the Python wrapper passes them, and
 Julia's D x M), the bad coordinate first, in the middle and last, in each
@@ -24,7 +25,8 @@ CASES = {
     "image": ((64, 48), 900, True),
     "manytiles": ((1100, 1200), 3000, True),  # 138 x 150 tiles of 16^2
     "volume": ((24, 20, 28), 800, True),
-    "nodeparallel": ((8, 7), 500, False),
+    "nodeparallel": ((8, 7), 500, False),      # looked at on the host
+    "nodeparallel_many": ((8, 7), 5000, False),
 }
 
 
