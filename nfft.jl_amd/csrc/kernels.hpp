@@ -303,6 +303,28 @@ __device__ __forceinline__ double dpp_rows(double v) {
   u.y = __builtin_amdgcn_update_dpp(0, u.y, CTRL, ROWMASK, 0xF, false);
   return *reinterpret_cast<double*>(&u);
 }
+// Lane L of each aligned group of G lanes (2, 4, 8 or 16; L < G), in all lanes of
+// the group: quad permutation, or a broadcast within rows of 16 (in two halves
+// for G = 8).
+template <int G, int L>
+__device__ __forceinline__ int group_lane(int v) {
+  if constexpr (G <= 4) {
+    constexpr int q = G == 4 ? L * 0x55 : L * 0x55 + 0xA0;  // quad_perm(L, L, L, L) or (L, L, 2 + L, 2 + L)
+    return __builtin_amdgcn_update_dpp(0, v, q, 0xF, 0xF, false);
+  } else {
+    const int u = __builtin_amdgcn_update_dpp(0, v, 0x150 + L, 0xF, 0xF, false);  // row_newbcast
+    if constexpr (G == 16) return u;
+    return __builtin_amdgcn_update_dpp(u, v, 0x150 + (L + 8) % 16, 0xF, 0xC, false);
+  }
+}
+template <int G, int L>
+__device__ __forceinline__ float group_lane(float v) {
+  return __int_as_float(group_lane<G, L>(__float_as_int(v)));
+}
+template <int G, int L>
+__device__ __forceinline__ double group_lane(double v) {
+  return __hiloint2double(group_lane<G, L>(__double2hiint(v)), group_lane<G, L>(__double2loint(v)));
+}
 __device__ __forceinline__ float readlane(float v, int l) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
@@ -426,9 +448,16 @@ __global__ __launch_bounds__(256) void k_node_records(KArgs a, char* __restrict_
 // groups consecutive records.  (Copying the records through LDS took a block
 // copy, a barrier and, per node, as many LDS reads as the taps have adds; two
 // or four steps ahead: more registers, the same or a longer time.)
-template <typename R, int D, int W>
+// OWN (interpolation with more than 32 bytes of dimension-2 weights): one of
+// them per lane, passed round the group (group_lane), where all W in every lane
+// bound crowded tiles by the loads: 256^2, 16 nodes per pixel, us of
+// interpolation, FP64 m = 3 43 -> 40, m = 5 88 -> 77, FP32 m = 5 49 -> 47
+// (records through LDS: 39, 76, 47).  FP32 m = 4 is no faster by it alone and
+// slower in a batch (165 -> 176).
+template <typename R, int D, int W, bool OWN = false>
 struct NodeTaps {
-  R w1, w2[D == 2 ? W : 1];
+  static constexpr int N2 = D == 2 && !OWN ? W : 1;
+  R w1, w2[N2];
   unsigned pk;
   int pj;
   __device__ __forceinline__ void load(const char* __restrict__ rec, long long j, int lx) {
@@ -437,13 +466,26 @@ struct NodeTaps {
     w1 = ((const R*)r)[lx];
     if constexpr (D == 2) {
 #pragma unroll
-      for (int l = 0; l < W; ++l) w2[l] = ((const R*)r)[W + l];
+      for (int l = 0; l < N2; ++l) w2[l] = ((const R*)r)[W + (OWN ? lx : l)];
     }
     const int2 q = *(const int2*)(r + N::WBYTES);
     pk = (unsigned)q.x;
     pj = q.y;
   }
 };
+
+// Taps of one column of a node's footprint: rows L .. W - 1, the weight of row
+// L from lane L of the group.
+template <int L, int W, int G, typename R, typename C>
+__device__ __forceinline__ void interp_rows(const C* col, int Sx, R w2, R* ar, R* ai) {
+  if constexpr (L < W) {
+    const R w = group_lane<G, L>(w2);
+    const C v = col[Sx * L];
+    *ar = fma(w, v.x, *ar);
+    *ai = fma(w, v.y, *ai);
+    interp_rows<L + 1, W, G>(col, Sx, w2, ar, ai);
+  }
+}
 
 // Fields of a record in LDS.
 template <typename R, int D, int W>
@@ -829,7 +871,8 @@ __device__ __forceinline__ void interp_tile_item(const KArgs& a, int item,
   C* tile = (C*)smem;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int slot = lane / G, lx = lane & (G - 1), lw = min(lx, W - 1);
-  NodeTaps<R, D, W> nx;
+  constexpr bool OWN = D == 2 && W * sizeof(R) > 32;
+  NodeTaps<R, D, W, OWN> nx;
   {
     const int n = it.y + wave * NPW + slot;
     nx.load(a.rec, n < it.z ? n : it.y, lw);
@@ -876,7 +919,7 @@ __device__ __forceinline__ void interp_tile_item(const KArgs& a, int item,
   for (int n0 = it.y + wave * NPW; n0 < it.z; n0 += NW * NPW) {
     const int n = n0 + slot;
     const bool on = n < it.z;
-    const NodeTaps<R, D, W> c = nx;
+    const NodeTaps<R, D, W, OWN> c = nx;
     R wold = 0;  // the weight to be divided, in flight during the taps
     if (D == 2 && a.wdiv && lx == 0 && on) wold = ((const C*)a.wdiv)[c.pj].x;
     const int m = n + NW * NPW;
@@ -885,11 +928,15 @@ __device__ __forceinline__ void interp_tile_item(const KArgs& a, int item,
     if (on && lx < W) {
       if constexpr (D == 2) {
         const int base = ((int)(c.pk & LM) + lx) + a.Sx * (int)(c.pk >> 16);
+        if constexpr (OWN) {
+          interp_rows<0, W, G>(tile + base, a.Sx, c.w2[0], &ar, &ai);
+        } else {
 #pragma unroll
-        for (int ly = 0; ly < W; ++ly) {
-          const C v = tile[base + a.Sx * ly];
-          ar = fma(c.w2[ly], v.x, ar);
-          ai = fma(c.w2[ly], v.y, ai);
+          for (int ly = 0; ly < W; ++ly) {
+            const C v = tile[base + a.Sx * ly];
+            ar = fma(c.w2[ly], v.x, ar);
+            ai = fma(c.w2[ly], v.y, ai);
+          }
         }
         ar *= c.w1;
         ai *= c.w1;
