@@ -868,6 +868,13 @@ __device__ __forceinline__ void interp_tile_item(const KArgs& a, int item,
   constexpr int NPW = 64 / G;
   extern __shared__ __align__(16) char smem[];
   const int4 it = a.items[item];
+  // a batch has its KArgs in global memory: fields used among the stores of the
+  // node loop are read once, here
+  const char* const rec = a.rec;
+  const long long fst = a.fst;
+  const int Sx = a.Sx;
+  C* const wdiv = (C*)a.wdiv;
+  int* const wbad = a.wbad;
   C* tile = (C*)smem;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int slot = lane / G, lx = lane & (G - 1), lw = min(lx, W - 1);
@@ -875,7 +882,7 @@ __device__ __forceinline__ void interp_tile_item(const KArgs& a, int item,
   NodeTaps<R, D, W, OWN> nx;
   {
     const int n = it.y + wave * NPW + slot;
-    nx.load(a.rec, n < it.z ? n : it.y, lw);
+    nx.load(rec, n < it.z ? n : it.y, lw);
   }
   int t0[3] = {0, 0, 0};
   tile_origin(a, D, it.x, t0);
@@ -915,25 +922,25 @@ __device__ __forceinline__ void interp_tile_item(const KArgs& a, int item,
   }
   __syncthreads();
 
-  const R osc = (R)a.oscale, gd = D == 2 && a.wdiv ? (R)a.gdiv[0] : (R)1;
+  const R osc = (R)a.oscale, gd = D == 2 && wdiv ? (R)a.gdiv[0] : (R)1;
   for (int n0 = it.y + wave * NPW; n0 < it.z; n0 += NW * NPW) {
     const int n = n0 + slot;
     const bool on = n < it.z;
     const NodeTaps<R, D, W, OWN> c = nx;
     R wold = 0;  // the weight to be divided, in flight during the taps
-    if (D == 2 && a.wdiv && lx == 0 && on) wold = ((const C*)a.wdiv)[c.pj].x;
+    if (D == 2 && wdiv && lx == 0 && on) wold = wdiv[c.pj].x;
     const int m = n + NW * NPW;
-    nx.load(a.rec, m < it.z ? m : it.y, lw);
+    nx.load(rec, m < it.z ? m : it.y, lw);
     R ar = 0, ai = 0;
     if (on && lx < W) {
       if constexpr (D == 2) {
-        const int base = ((int)(c.pk & LM) + lx) + a.Sx * (int)(c.pk >> 16);
+        const int base = ((int)(c.pk & LM) + lx) + Sx * (int)(c.pk >> 16);
         if constexpr (OWN) {
-          interp_rows<0, W, G>(tile + base, a.Sx, c.w2[0], &ar, &ai);
+          interp_rows<0, W, G>(tile + base, Sx, c.w2[0], &ar, &ai);
         } else {
 #pragma unroll
           for (int ly = 0; ly < W; ++ly) {
-            const C v = tile[base + a.Sx * ly];
+            const C v = tile[base + Sx * ly];
             ar = fma(c.w2[ly], v.x, ar);
             ai = fma(c.w2[ly], v.y, ai);
           }
@@ -949,12 +956,12 @@ __device__ __forceinline__ void interp_tile_item(const KArgs& a, int item,
     ar = group_sum<G>(ar);
     ai = group_sum<G>(ai);
     if (lx == 0 && on) {
-      if (D == 2 && a.wdiv) {
+      if (D == 2 && wdiv) {
         const R t = ar * osc / gd;
-        if (!(t > (R)0)) a.wbad[0] = 1;
-        ((C*)a.wdiv)[c.pj] = C{wold / t, (R)0};
+        if (!(t > (R)0)) wbad[0] = 1;
+        wdiv[c.pj] = C{wold / t, (R)0};
       } else {
-        fhat[(long long)c.pj * a.fst] = C{ar * osc, ai * osc};
+        fhat[(long long)c.pj * fst] = C{ar * osc, ai * osc};
       }
     }
   }
