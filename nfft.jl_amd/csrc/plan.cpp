@@ -1773,7 +1773,7 @@ struct nfftm_batch_s {
   bool called = false;
   hipEvent_t switch_ev = nullptr;  // orders calls on different streams
   struct TileGroup {
-    int D = 0, W = 0, NT = 0, nblk = 0, nwork = 0;
+    int D = 0, W = 0, NT = 0, nblk[2] = {0, 0}, nwork = 0;  // workgroups of interpolation and spreading
     size_t lds = 0;
     DevBuf<int2> work;
   };
@@ -1821,11 +1821,11 @@ int batch_enqueue(nfftm_batch_s& b, bool forward, hipStream_t s) {
     for (auto& g : b.fg)
       if (int rc = g.fft->exec(true, g.base, b.celem, s)) return rc;
     for (auto& g : b.tg)
-      HIPCHK(launch_tile_batch(g->D, false, b.dbl, g->W, g->NT, g->nblk, g->lds, s, b.d_ka.p, g->work.p, g->nwork,
+      HIPCHK(launch_tile_batch(g->D, false, b.dbl, g->W, g->NT, g->nblk[0], g->lds, s, b.d_ka.p, g->work.p, g->nwork,
                                (const void* const*)grids, tout));
   } else {
     for (auto& g : b.tg)
-      HIPCHK(launch_tile_batch(g->D, true, b.dbl, g->W, g->NT, g->nblk, g->lds, s, b.d_ka.p, g->work.p, g->nwork,
+      HIPCHK(launch_tile_batch(g->D, true, b.dbl, g->W, g->NT, g->nblk[1], g->lds, s, b.d_ka.p, g->work.p, g->nwork,
                                (const void* const*)tin, nullptr));
     for (int d = 0; d < 2; ++d)
       HIPCHK(launch_fold_batch(d + 1, b.dbl, b.fold[d].nblk, s, b.d_ka.p, b.fold[d].work.p, b.fold[d].nwork, grids));
@@ -1960,8 +1960,12 @@ int batch_build(nfftm_batch_s& b, const nfftm_plan* plans, const int* ntrans, in
     auto& G = *b.tg[g];
     if (int rc = upload(G.work, tw[g])) return rc;
     G.nwork = (int)tw[g].size();
-    G.nblk = std::min(tile_batch_blocks(G.D, false, b.dbl, G.W, G.NT, G.lds), ((G.nwork + 7) / 8) * 8);
-    G.nblk = std::max(G.nblk, 8);
+    // each kernel's own residency: a grid sized by the other's leaves a second,
+    // nearly empty round of workgroups or idle CUs (FP64, m = 5)
+    for (int d = 0; d < 2; ++d) {
+      const int res = tile_batch_blocks(G.D, d == 1, b.dbl, G.W, G.NT, G.lds);
+      G.nblk[d] = std::max(8, std::min(res, ((G.nwork + 7) / 8) * 8));
+    }
   }
   if (int rc = upload(b.dec.work, dec)) return rc;
   b.dec.nwork = (int)dec.size();
