@@ -1681,11 +1681,11 @@ int time_gridding(nfftm_plan_s& p, void* fh, double* ms) {
 }
 
 // Candidate shapes: D = 2 tile edges 16..128, D = 1 edges 512..8192, with 256
-// or 512 threads (maxNT caps it); D = 3: both compile-time geometries with 512
+// or 512 threads (minNT .. maxNT); D = 3: both compile-time geometries with 512
 // or 1024 threads.  Plans of more than 2^20 nodes are timed on every k-th node
 // (the same spatial distribution at a bounded binning cost); the nodes are
 // binned once per geometry.  Leaves the fastest applied to all nodes.
-int tune_plan(nfftm_plan_s& p, int maxNT, std::vector<TuneChoice>* log) {
+int tune_plan(nfftm_plan_s& p, int minNT, int maxNT, std::vector<TuneChoice>* log) {
   if (!p.tiled || p.M == 0) return NFFTM_OK;
   const i64 Mfull = p.M;
   std::vector<double> kfull;
@@ -1710,7 +1710,7 @@ int tune_plan(nfftm_plan_s& p, int maxNT, std::vector<TuneChoice>* log) {
                                          : std::vector<int>{512, 1024, 2048, 4096, 8192};
     for (int t : ts)
       for (int nt : {256, 512})
-        if (nt <= maxNT) cand.push_back({t, nt});
+        if (nt >= minNT && nt <= maxNT) cand.push_back({t, nt});
   }
   TuneChoice best;
   best.ms = 1e30;
@@ -1861,7 +1861,11 @@ int batch_build(nfftm_batch_s& b, const nfftm_plan* plans, const int* ntrans, in
   b.S = (int)b.slot_plan.size();
   if (flags & NFFTM_BATCH_AUTOTUNE)
     for (auto* p : b.plans)
-      if (int rc = tune_plan(*p, 512, nullptr)) return rc;
+      // plans of another workgroup size are another launch after the first: in
+      // FP64 the two take longer than one with 512 throughout (16 plans and 8
+      // images, m = 5: forward 654 -> 594 us, adjoint 895 -> 853; m = 3, 4 the same;
+      // FP32 m = 3: 230 -> 242, 306 -> 329)
+      if (int rc = tune_plan(*p, b.dbl ? 512 : 256, 512, nullptr)) return rc;
   for (auto* p : b.plans) {
     // the batch kernels read node records, which 1-D polynomial-window plans
     // do not keep for themselves
@@ -2540,7 +2544,7 @@ int nfftm_binning(nfftm_plan p, int* nitems, int32_t* perm_host, int32_t* items_
 int nfftm_plan_tune(nfftm_plan p) {
   g_err.clear();
   if (!p) return fail(NFFTM_ERR_ARG, "plan is NULL");
-  return tune_plan(*p, 1024, nullptr);
+  return tune_plan(*p, 256, 1024, nullptr);
 }
 
 int nfftm_plan_set_tiles(nfftm_plan p, int tile, int threads) {
