@@ -509,7 +509,7 @@ double best_threads(int L, const int* r, int n, int most, int* tpl) {
 
 // The radices of a line of L points: least cost.
 struct Search {
-  int L, most;
+  int L, most, rmax;
   int cur[MIX_PASSES], best[MIX_PASSES], nb, tpl;
   double cost;
   void go(int n, int nc) {
@@ -526,7 +526,7 @@ struct Search {
     }
     if (nc >= MIX_PASSES) return;
     for (int r : RADICES)
-      if (n % r == 0 && (nc == 0 || r <= cur[nc - 1])) {
+      if (n % r == 0 && r <= (nc == 0 ? rmax : cur[nc - 1])) {
         cur[nc] = r;
         go(n / r, nc + 1);
       }
@@ -539,11 +539,12 @@ constexpr int max_points(bool dbl) { return dbl ? 8192 : 16384; }
 
 }  // namespace
 
-bool mix_factor(int64_t L, bool dbl, bool only, MixLine* ln) {
+bool mix_factor(int64_t L, bool dbl, bool only, MixLine* ln, int rmax) {
   // the strided passes want rows of at least 32 bytes within the LDS
   if (L < 16 || L % 2 || L > (only ? max_points(dbl) / 2 : 2048)) return false;
   Search se;
   se.L = (int)L;
+  se.rmax = rmax;
   se.most = max_threads(dbl) / (only ? 1 : dbl ? 2 : 4);
   se.cost = 1e30;
   se.go(se.L, 0);

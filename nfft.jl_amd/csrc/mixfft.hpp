@@ -62,8 +62,9 @@ struct MixArgs {
 };
 
 // Radices of a line of L points; false where the passes are not built for it
-// (only: the line is the whole 1-D grid, no strided pass follows).
-bool mix_factor(int64_t L, bool dbl, bool only, MixLine* ln);
+// (only: the line is the whole 1-D grid, no strided pass follows; rmax: largest
+// radix).
+bool mix_factor(int64_t L, bool dbl, bool only, MixLine* ln, int rmax = 16);
 // Lines per workgroup of the dimension-1 pass (col = false) or of a strided
 // pass, for `lines` lines at each of `outer` positions.
 int mix_shape(bool dbl, bool col, const MixLine& ln, long long lines, long long outer);

@@ -2811,7 +2811,13 @@ int nfftm_toeplitz_create(nfftm_toeplitz* out, int prec, int D, const int64_t* N
   t->fft.reset(new FFTStage());
   if (int rc = t->fft->build(D, t->L, t->dbl())) return rc;
   t->mix = D >= 2 && t->Q < (1LL << 31);
-  for (int d = 0; d < D && t->mix; ++d) t->mix = mix_factor(t->L[d], t->dbl(), false, &t->ln[d]);
+  // Up to 256^2 points in 2-D the three launches take the time of one line each:
+  // without radix 16, whose butterfly is a long chain (us, FP32 / FP64: 128^2
+  // image 26.0 -> 21.9 / 27.5 -> 22.7, rocFFT 20.4 / 21.3; 48^2 24.0 -> 20.2 / 24.7
+  // -> 20.2, rocFFT 28.0 / 21.1).  Larger ones are better with it (512^2 image: 30.6
+  // against 32.2 / 49.7 against 55.9).
+  const int rmax = D == 2 && t->Q <= 65536 ? 13 : 16;
+  for (int d = 0; d < D && t->mix; ++d) t->mix = mix_factor(t->L[d], t->dbl(), false, &t->ln[d], rmax);
   if (t->mix) {
     std::vector<char> h;
     for (int d = 0; d < D; ++d) {

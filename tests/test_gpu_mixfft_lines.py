@@ -6,8 +6,8 @@ grid and 4096 of an FP64 one (a whole workgroup on one line), strided and
 dimension-1 lines of up to 2048 points beside short axes, in 2-D and 3-D.  The
 plans are directional with one slice, so that forward and adjoint of both
 precisions take the passes.  Toeplitz products on both sides of the sizes whose
-last-dimension pass (two lines' LDS areas) no longer fits the LDS, against FFTs
-of the padded image in FP64.
+last-dimension pass (two lines' LDS areas) no longer fits the LDS, and of those
+whose lines are taken without radix 16, against FFTs of the padded image in FP64.
 """
 import numpy as np
 import pytest
@@ -75,6 +75,7 @@ def test_lines(N, dtype):
 # Lines of 2 n points along the last (first Python) dimension.  Short rest axes
 # give the fewest lines per workgroup (FP64 2, FP32 4), the long ones 8 or 4.
 TOEP = [(n, r) for r in [(9,), (6, 5)] for n in (500, 693, 728, 735, 924, 936, 1024)]
+TOEP += [(128, (128,)), (48, (56,)), (8, (64,)), (128, (129,))]  # up to 256^2 points and above
 TOEP += [(n, (40, 60)) for n in (264, 273, 462, 468, 528, 539, 546, 600, 1024)]
 
 
