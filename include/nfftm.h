@@ -80,7 +80,13 @@ enum {
                               deconvolution fused; on 1-D grids of n1 Lm^2
                               points (Lm = 64, 128, 256; n1 = 2^k or 5 2^k):
                               three passes of line FFTs, deconvolution
-                              fused.  Results agree to rounding;
+                              fused; on other grids of prime factors up to 13
+                              (2048 points per dimension, a 1-D grid 8192 in
+                              FP32 and 4096 in FP64; D <= 3) the pruned line
+                              FFTs with radices chosen per plan, where an FP32
+                              plan that is not directional takes them in the
+                              adjoint only (its forward grid gives the FP64
+                              node gradient).  Results agree to rounding;
                               the grid (nfftm_grid) then holds the full FFT
                               after a forward transform and a partial one
                               after an adjoint. */
@@ -215,7 +221,8 @@ int nfftm_fft(nfftm_plan p, void* g_dev, int direction);
  * (src/precomputation.jl:25-29). */
 int nfftm_sizes(nfftm_plan p, int64_t* Ntilde, int64_t* M, double* sigma);
 
-/* The plan's internal grid (p.tmpVec) as a device pointer. */
+/* The plan's internal grid (p.tmpVec) as a device pointer; what it holds after
+ * a transform: NFFTM_FLAG_ROCFFT. */
 int nfftm_grid(nfftm_plan p, void** g_dev);
 
 /* TimingStats fields (AbstractNFFTs/src/misc.jl:22-30), seconds:

@@ -7,21 +7,24 @@
 // are Stockham passes in LDS whose radices come from a per-plan list
 // (MixLine) instead of template parameters.  A pass branches once, on a
 // uniform radix, to code for that radix; a thread holds all butterflies it
-// owns (16 points, rounded up to whole butterflies) in registers between the
+// owns (8 points, rounded up to whole butterflies) in registers between the
 // reads and the writes of a pass, so that one LDS copy of the lines suffices.
 // The first pass takes its points from global memory and the last one
 // writes its results there.  Divisions are by multiply-high.
 //
 // What bounds it: HBM where the grid exceeds the caches (the LDS work of a
 // line of 3 passes is about a third of its HBM time); the line latency on
-// small images, hence few lines per workgroup there (mix_lines_per_block).
+// small images, hence few lines per workgroup there (mix_shape).
 // The radices and the threads per line are those with the fewest exchanges
 // and idle butterfly slots (best_threads); lines with a prime factor above 13
 // keep rocFFT.
 //
-// Measured (us of the whole FFT stage with the deconvolution, forward +
-// adjoint; rocFFT with separate deconvolution before): 300 x 288 x 250 FP32
-// 1077 -> 305, 192^3 FP64 340 -> 160, 640^2 FP64 92 -> 49, 480^2 FP32 50 -> 40.
+// Measured (us of the whole FFT stage with the deconvolution, forward /
+// adjoint, against rocFFT with separate deconvolution): 300 x 288 x 250 FP32
+// 129 / 119 against 495 / 477, 192^3 FP64 72 / 71 against 179 / 169, 640^2 FP64
+// 23 / 22 against 37 / 36, 32 slices of 480^2 FP32 53 / 50 against 896 / 870.
+// (Ordinary FP32 plans keep rocFFT in the forward direction: plan.cpp,
+// mix_forward.)
 //
 // Lines of the strided passes are lpb consecutive x positions: every load and
 // store row is a contiguous run of lpb elements.  Rows of a grid whose width

@@ -913,8 +913,9 @@ hipError_t launch_slot_sum(bool dbl, const KArgs& a, size_t slot_bytes, const in
 }
 
 // Adjoint with the fold fused into the first pruned FFT pass (lines along
-// dimension 3, inverse FFT, output kept on S_z), for grids of whole tiles, one
-// slot per tile (k_slot_sum).  Workgroup (ox, y) takes the T lines x of tile
+// dimension 3, inverse FFT, output kept on S_z), for grids of whole tiles that
+// hold one work item each at most (crowded tiles take k_slot_sum and the
+// separate fold: fused_fold in plan.cpp).  Workgroup (ox, y) takes the T lines x of tile
 // column ox at row y (E / L = T lines of L points); thread (lx, j0) sums its
 // 16 points z = j0 + u L / 16 from the slots exactly as k_fold3b sums them
 // (same neighbours in the same order, so the grid values are bit-identical),

@@ -783,8 +783,8 @@ __global__ __launch_bounds__(256) void k_fold(KArgs a, typename cpx<R>::T* __res
 // 2-D fold where every tile has at least m cells per dimension: a point is
 // covered by its own tile and the eight around it only.  One workgroup per
 // tile, a thread per point: the item ranges of the nine tiles are uniform and
-// read together, then the (at most four) covering values together, where
-// fold_sum walks the covering pairs one dependent load after the other
+// read together, then the covering values together (four at most where the
+// tiles have 2m - 1 cells or more, up to nine on smaller ones), where fold_sum walks the covering pairs one dependent load after the other
 // (512^2 points, FP32, radial nodes: 12.9 -> 9 us).
 template <typename R>
 __device__ __forceinline__ void fold2_point(const KArgs& a, const typename cpx<R>::T* __restrict__ scr,

@@ -2,10 +2,11 @@
 whole-grid rocFFT stage and the oracle.
 
 Grids that are not powers of two: FP64 rel-l2 <= 1e-13 between the two paths
-and <= 1e-12 against the CPU oracle; FP32 <= 2e-6 between the paths.  The
-sizes cover every radix of the list, lines of one to five passes, the largest
-lines of each precision, few and many lines per workgroup and ragged chunks
-of lines.
+and <= 1e-12 against the CPU oracle; FP32 <= 2e-6 between the paths (forward
+transforms of FP32 plans that are not directional run rocFFT themselves).  The
+sizes cover every radix of the list, lines of two to four passes, few and many
+lines per workgroup, ragged chunks of lines and a grid that stays with rocFFT
+(302 = 2 151); the ends of the range are in test_gpu_mixfft_lines.py.
 """
 import numpy as np
 import pytest
@@ -34,7 +35,7 @@ CASES = [
     ((13, 11), 2.0),          # 26 = 2 13, 22 = 2 11
     ((10, 24), 2.0),          # 20, 48
     ((75, 96), 2.0),          # 150, 192
-    ((250, 37), 1.21),        # 302 = 2 151 (rocFFT) beside 44 = 4 11
+    ((250, 37), 1.21),        # 302 = 2 151 beside 44: rocFFT for both
     ((320, 45), 2.0),         # 640, 90
     ((81, 147), 2.0),         # 162, 294 = 2 3 7 7
     ((700, 20), 2.0),         # 1400 = 2^3 5^2 7

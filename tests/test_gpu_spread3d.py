@@ -36,7 +36,7 @@ def test_widths(m, nodes):
     N = (20, 17, 18)
     if nodes == "sparse":
         k = rng.random((3, 301)) - 0.5
-    else:  # a few crowded tiles: batches of 128 or 256, items of 1024
+    else:  # a few crowded tiles: several batches of an item, items of 1024
         k = 0.2 * (rng.random((3, 3001)) - 0.5) + 0.1
     p, d, want = check(k, N, m)
     for variant in (0, 1):
