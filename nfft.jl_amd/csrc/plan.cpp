@@ -1078,17 +1078,24 @@ int set_nodes(nfftm_plan_s& p, const double* k, bool rows, i64 M, bool keep) {
   nfftm_plan_s::BinWork& w = p.bw;
   struct Release {
     nfftm_plan_s& p;
-    bool keep;
+    bool keep, read;  // read: the caller's nodes have been copied
     ~Release() {
-      if (keep) return;
-      (void)hipStreamSynchronize(p.stream);  // the kernels that use them
-      p.bw.release();
+      // the copy out of the caller's array (a failure in between), the kernels
+      // that use the work arrays
+      if (!keep || !read) (void)hipStreamSynchronize(p.stream);
+      if (!keep) p.bw.release();
     }
-  } release{p, keep};
+  } release{p, keep, false};
   // The node arrays are rewritten in place, and the plan's own stream is not
   // the only one that reads them: a batch holds their addresses and runs on its
   // caller's.  (gen = 0: a plan under construction, nothing reads it yet.)
   if (p.gen > 0) HIPCHK(hipDeviceSynchronize());
+  // node-parallel plans run no binning kernel that looks at the nodes: a few
+  // nodes are looked at here, before anything reads them (for 200 of them the
+  // kernel, its flag's fill and copy took 7 of 43 us), the plan's own need no look
+  const bool seen = !p.tiled && (!k || (i64)D * M <= 4096);
+  if (seen && k)
+    if (int rc = check_nodes(k, (i64)D * M)) return rc;
   if (k) {
     HIPCHK(w.k.ensure((size_t)D * M));
     if (M) HIPCHK(hipMemcpyAsync(w.k.p, k, (size_t)D * M * sizeof(double), hipMemcpyHostToDevice, st));
@@ -1131,12 +1138,6 @@ int set_nodes(nfftm_plan_s& p, const double* k, bool rows, i64 M, bool keep) {
   a.key_bits = 1;
   while (((i64)1 << a.key_bits) < ntile) ++a.key_bits;
   int nitems = 0, nmulti = 0;
-  // node-parallel plans run no binning kernel that looks at the nodes: a few
-  // nodes are looked at here (for 200 of them the kernel, its flag's fill and
-  // copy took 7 of 43 us), the plan's own need no look
-  const bool seen = !p.tiled && (!k || (i64)D * M <= 4096);
-  if (seen && k)
-    if (int rc = check_nodes(k, (i64)D * M)) return rc;
   HIPCHK(w.stats.ensure(4));
   // pinned where nodes! comes again (its allocation costs a plan more than it saves once)
   int hs[4] = {0, 0, 0, 0}, *hp = hs;
@@ -1158,6 +1159,7 @@ int set_nodes(nfftm_plan_s& p, const double* k, bool rows, i64 M, bool keep) {
   }
   if (!seen) HIPCHK(hipMemcpyAsync(hp, w.stats.p, 4 * sizeof(int), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
+  release.read = true;
   if (!seen && hp[3]) return bad_node();
   if (p.tiled) {
     nitems = hp[0];
