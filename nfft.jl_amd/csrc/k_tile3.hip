@@ -1022,7 +1022,7 @@ static hipError_t fold_fft3_l(const KArgs& a, const FArgs& f, hipStream_t s, voi
 
 template <typename R, int W>
 static hipError_t fold_fft3_v(const KArgs& a, const FArgs& f, hipStream_t s, void* grid, bool dry) {
-  if (a.tvar == 2) return hipErrorNotSupported;  // lines of at least 128 points hold the long tile
+  if (a.tvar == 2) return hipErrorNotSupported;  // on such lines the tile of plans with few nodes
   return a.tvar ? fold_fft3_l<R, W, 1>(a, f, s, grid, dry) : fold_fft3_l<R, W, 0>(a, f, s, grid, dry);
 }
 

@@ -892,15 +892,17 @@ bool tiles_ok(const nfftm_plan_s& p);
 // Whether variant 0 of a width with a long tile (FP64, 2m = 10: 8 x 8 x 16)
 // takes the cubic one (8^3): where the grid does not hold the long tile's
 // padded edge (it would be left to the node-parallel kernels: 9 .. 12 slices
-// of 96^2, 2 10^5 nodes: adjoint 18.3 ms instead of 0.2), and below 1024 long
-// tiles, which leave most of the chip idle (sigma = 2, us of interpolation +
-// spreading with the fold, cubic / long: 24^3 image, 200 nodes 34 / 52, 5 10^4
-// nodes 77 / 149; 48^3, 864 long tiles, 36 / 55, 124 / 127; 64^3, 2048 of
-// them, 36 / 46, 277 / 199).
+// of 96^2, 2 10^5 nodes: adjoint 18.3 ms instead of 0.2), on grids of less than
+// 1024 long tiles in volume, which leave most of the chip idle (sigma = 2, us of
+// interpolation + spreading with the fold, cubic / long: 24^3 image, 200 nodes
+// 34 / 52, 5 10^4 nodes 77 / 149; 48^3, 864 long tiles, 36 / 55, 124 / 127; 64^3,
+// 2048 of them, 277 / 199), and where the plan is made for no more nodes than
+// long tiles, whose items are mostly their slots (adjoint, 64^3 image: 1000 nodes
+// 66 / 83, 2000 86 / 97, 4000 112 / 110; 96^3, 6900 nodes 315 / 365; 128^3, 8000
+// nodes 485 / 512, 16000 707 / 695; forward transforms up to 7 % shorter as well).
 bool short_tile3(const nfftm_plan_s& p, const int* T, const int* P) {
-  i64 n = 1;
-  for (int d = 0; d < 3; ++d) n *= (p.Nt[d] + T[d == 2] - 1) / T[d == 2];
-  return p.Nt[2] < P[1] || n < 1024;
+  const i64 n = p.Nt[0] * p.Nt[1] * p.Nt[2] / ((i64)T[0] * T[0] * T[1]);
+  return p.Nt[2] < P[1] || n < 1024 || p.M <= n;
 }
 
 // 3-D geometry of variant V (compile-time tile of k_tile3.hip); false if

@@ -1,6 +1,7 @@
 """Tile edge along dimension 3 of FP64 plans with 2m = 10: 8 x 8 x 16 cells, or
-8^3 where the grid is shorter than the long tile's padded edge (25 cells) or
-has fewer than 1024 long tiles.
+8^3 where the grid is shorter than the long tile's padded edge (25 cells), has
+the volume of fewer than 1024 long tiles, or the plan is made for no more nodes
+than long tiles.
 
 Every grid that holds the cubic tile's padded edge (17 cells) is tiled, and
 forward and adjoint equal the oracle (FP64 rel-l2 <= 1e-12) on both sides of
@@ -80,3 +81,36 @@ def test_lines():
         assert plan((24, 24, 24), 300, m, dtype)[1].tile_shape()[1] == 1024
     _, p = plan((8, 30, 30), 300)    # 16 cells: node-parallel, as before
     assert p.tile_shape()[0] == (0, 0, 0)
+
+
+@pytest.mark.parametrize("N,n", [((64, 64, 64), 2048), ((50, 50, 53), 1035)], ids=["whole", "ragged"])
+def test_few_nodes(N, n):
+    """Up to n nodes, n the volume of the grid in long tiles: the cubic tile, also
+    on power-of-two grids (separate fold); one more: the long one.  nodes!
+    keeps the tile, copy and set_tiles choose for the nodes there are."""
+    print(f"short tile, few nodes N={N}", flush=True)
+
+    def check(p, k):
+        M = k.shape[1]
+        q = nfftm.plan_nfft(k, N, m=5, sigma=2.0, precompute=nfftm.LINEAR, sparse_matrix=True)
+        f = torch.randn(N, dtype=torch.complex128, device="cuda")
+        fh = torch.randn(M, dtype=torch.complex128, device="cuda")
+        assert O.relerr((p * f).cpu().numpy(), (q * f).cpu().numpy()) < 1e-13
+        assert O.relerr((p.H * fh).cpu().numpy(), (q.H * fh).cpu().numpy()) < 1e-13
+
+    ka, a = plan(N, n)
+    kb, b = plan(N, n + 1)
+    assert a.tile_shape()[0] == (8, 8, 8) and b.tile_shape()[0] == (16, 8, 8)
+    check(a, ka)
+    check(b, kb)
+    a.nodes_(kb)
+    b.nodes_(ka)
+    assert a.tile_shape()[0] == (8, 8, 8) and b.tile_shape()[0] == (16, 8, 8)
+    check(a, kb)
+    check(b, ka)
+    c = a.copy()
+    assert c.tile_shape()[0] == (16, 8, 8)
+    check(c, kb)
+    b.set_tiles(0, 1024)
+    assert b.tile_shape()[0] == (8, 8, 8)
+    check(b, ka)
