@@ -856,6 +856,15 @@ __global__ __launch_bounds__(256) void k_fold2(KArgs a, typename cpx<R>::T* __re
 // every node with G lanes per node (one per dimension-1 column); the first
 // records are read while the tile is staged, each later one a step ahead
 // (32 slices of 1.2 10^5 nodes, FP32, m = 4: 130 -> 121 us).
+//
+// Every lane of a group has the sums of its node: lane s keeps those of step s,
+// and the lanes store together after KEEP steps, ahead of the next loads.  With a
+// store in every step each wait for a record, which counts stores as well, was
+// one for the store just issued (us of interpolation: 100^2 image, 50 nodes per
+// pixel, FP32 m = 3 26.8 -> 20.8, m = 5 49 -> 42, FP64 m = 3 36 -> 33; 64^2, 50 per
+// pixel, FP64 m = 5 53 -> 41; 256^2, 16 per pixel, FP64 m = 3 39.0 -> 35.5).  FP32
+// keeps four: eight scattered stores of a group together took longer where the
+// results exceed the caches (256^2, 4 10^6 nodes, m = 4: 149 against 143).
 template <typename R, int D, int W, int NT>
 __device__ __forceinline__ void interp_tile_item(const KArgs& a, int item,
                                                  const typename cpx<R>::T* __restrict__ grid,
@@ -923,12 +932,30 @@ __device__ __forceinline__ void interp_tile_item(const KArgs& a, int item,
   __syncthreads();
 
   const R osc = (R)a.oscale, gd = D == 2 && wdiv ? (R)a.gdiv[0] : (R)1;
+  R kr = 0, ki = 0;  // the lane's results and their index (-1: none)
+  int kj = -1, step = 0;
+  constexpr int KEEP = sizeof(R) == 4 && G > 4 ? 4 : G;
+  auto store = [&]() {
+    if (kj < 0) return;
+    C* o = fhat + (long long)kj * fst;
+    C v{kr * osc, ki * osc};
+    if (D == 2 && wdiv) {
+      const R t = v.x / gd;
+      if (!(t > (R)0)) wbad[0] = 1;
+      o = wdiv + kj;
+      v = C{o->x / t, (R)0};
+    }
+    *o = v;
+    kj = -1;
+  };
   for (int n0 = it.y + wave * NPW; n0 < it.z; n0 += NW * NPW) {
     const int n = n0 + slot;
     const bool on = n < it.z;
     const NodeTaps<R, D, W, OWN> c = nx;
-    R wold = 0;  // the weight to be divided, in flight during the taps
-    if (D == 2 && wdiv && lx == 0 && on) wold = wdiv[c.pj].x;
+    if (step == KEEP) {
+      store();
+      step = 0;
+    }
     const int m = n + NW * NPW;
     nx.load(rec, m < it.z ? m : it.y, lw);
     R ar = 0, ai = 0;
@@ -955,16 +982,14 @@ __device__ __forceinline__ void interp_tile_item(const KArgs& a, int item,
     }
     ar = group_sum<G>(ar);
     ai = group_sum<G>(ai);
-    if (lx == 0 && on) {
-      if (D == 2 && wdiv) {
-        const R t = ar * osc / gd;
-        if (!(t > (R)0)) wbad[0] = 1;
-        wdiv[c.pj] = C{wold / t, (R)0};
-      } else {
-        fhat[(long long)c.pj * fst] = C{ar * osc, ai * osc};
-      }
+    if (lx == step && on) {
+      kr = ar;
+      ki = ai;
+      kj = c.pj;
     }
+    ++step;
   }
+  store();
 }
 
 template <typename R, int D, int W, int NT>
